@@ -118,6 +118,30 @@ def test_decode_matches_oracle_in_every_chunk_position(dt, D, H, Hkv):
         print(f"[result] dca decode dtype {dt} M={M}: max err {e:.2e}", flush=True)
 
 
+@pytest.mark.parametrize("dt,D,H,Hkv", [(orc.BF16, 128, 6, 6), (orc.F16, 128, 5, 1), (orc.BF16, 64, 12, 2),
+                                        (orc.BF16, 128, 16, 2), (orc.F16, 64, 16, 1), (orc.BF16, 128, 32, 2),
+                                        (orc.F32, 64, 12, 2), (orc.F32, 128, 16, 1)])
+def test_decode_group_sizes_and_block_edges(dt, D, H, Hkv):
+    """Every operand count of the 16-bit scores (3 H / Hkv columns in 16s), every group width of the
+    P.V kernel, caches that end at and beside a 256-key block, chunk edges off the 16-key tiles, and
+    token-major cache rows; bounds as in the test above."""
+    import _sta_native as native
+    s, w = 130, 33                                         # L = 97
+    g = torch.Generator().manual_seed(53 + dt + H)
+    for M in (1, 16, 255, 256, 257, 1283):
+        say(f"dca decode groups dtype {dt} D={D} H={H} Hkv={Hkv} M={M}")
+        q = (torch.randn(H, D, generator=g) * 2).to(TDT[dt]).to(DEV)
+        k = (torch.randn(M, Hkv, D, generator=g) * 2).to(TDT[dt]).to(DEV).transpose(0, 1)
+        v = torch.randn(M, Hkv, D, generator=g).to(TDT[dt]).to(DEV).transpose(0, 1)
+        out = native.dca_decode(q, k, v, _inv_freq(D), s, w, 1.0254)
+        torch.cuda.synchronize()
+        qn, odt = np_of(q)
+        kn, _ = np_of(k.contiguous())
+        vn, _ = np_of(v.contiguous())
+        ref = orc.dca_decode(qn, kn, vn, odt, _inv_freq(D).numpy(), s, w, np.float32(1.0254))
+        ulp_close(out.float().cpu().numpy(), ref, dt, f"groups M={M}", vmax=float(v.float().abs().max()))
+
+
 def test_decode_matches_reference_goldens():
     import _sta_native as native
     g = np.load(os.path.join(GOLD, "dca_decode_golden.npz"), allow_pickle=False)
