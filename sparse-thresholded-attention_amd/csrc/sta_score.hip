@@ -358,11 +358,18 @@ void score_kernel(ScoreArgs a) {
   __shared__ u32x4 lds[NBUF][LDS_UNITS];
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform: SGPR addresses
   // +inf hidden from the optimiser: med3(x, y, pinf) = max(x, y) stays one v_med3_f32, where a
   // literal +inf is rewritten into a max with two canonicalisations
   float pinf = INFINITY;
   asm volatile("" : "+s"(pinf));
+  // a value held per wave row (lane = row), read for an accumulator slot whose rows are r0 in lanes
+  // 0-31 and r0 + 4 in lanes 32-63
+  auto row_value = [&](float x, int r0) {
+    const float lo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), r0));
+    const float hi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), r0 + 4));
+    return lane < 32 ? lo : hi;
+  };
   const int rows_total = a.nt * T;               // == q_rows_pad
   const int ngroups = (rows_total + WG_ROWS - 1) / WG_ROWS;
   int h, g;
@@ -695,12 +702,11 @@ void score_kernel(ScoreArgs a) {
   // wave-uniform chunk bases in SGPRs and one lane offset: per-lane 64-bit addresses would hold
   // VGPRs through the sweep
   const uint32_t loff_h = (uint32_t)lane * 16u;
-  const int wave_s = __builtin_amdgcn_readfirstlane(wave);
   auto issue_hi = [&](int c, u32x4* dst) {
     const u32x4* src = kbase + (int64_t)c * CHUNK_UNITS;
 #pragma unroll
     for (int e = 0; e < LOADS_H; ++e) {
-      const int b = e * NW + wave_s;           // (32-key block, k step) b: its hi units, packed
+      const int b = e * NW + wave;           // (32-key block, k step) b: its hi units, packed
       copy16_to_lds_s(src + 128 * b, loff_h, lds_addr(dst + 64 * b));
     }
   };
@@ -919,9 +925,7 @@ void score_kernel(ScoreArgs a) {
           const float v = row32_max(t1[rb][i]);
           const int row = rb * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
           const int r0 = rb * 32 + (i >> 2) * 8 + (i & 3);     // the row of lanes 0-31; lanes 32-63: + 4
-          const float e0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ebase), r0));
-          const float e1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ebase), r0 + 4));
-          const float E = (lane < 32 ? e0 : e1) + 0x1p-20f * fabsf(v);
+          const float E = row_value(ebase, r0) + 0x1p-20f * fabsf(v);
           const float th = v - 2.0f * E;
           // padded rows never vote: their maximum is unused (no value reaches +inf)
           const bool valid = wrow0 + row < a.N;
@@ -1109,8 +1113,10 @@ void score_kernel(ScoreArgs a) {
     return false;
   };
 
-  // row max over the 32 lanes holding a row's keys (mx: the raw dot's running max per row slot),
-  // then the keep threshold x0 on the raw dot, and the weighted-vote origins.
+  // The keep threshold x0 on the raw dot and the weighted-vote origin of every row, from its raw
+  // maximum v, computed once per row by the row's lane (wave row `lane`) and read back into the 32
+  // row slots of each lane (min_arg_for's division and nextafter steps on every slot cost each wave
+  // 32 times as many: 15 us of a call on 8 heads x 2048 rows, fp32, 216 -> 201 us).
   // screened: the maximum came from the screen's four-product fp32 scores of the (hi + lo)
   // operands, which differ from pass 2's three-product value of the same key by the lo.lo term
   // and the two summation orders.  For tau >= 0 the threshold is then capped at max - delta, with delta a
@@ -1118,35 +1124,50 @@ void score_kernel(ScoreArgs a) {
   // share one dot, exact_2.py:100, 118, so qk == m passes whenever tau >= 0); for tau above
   // delta * scale (1e-5 at unit-scale rows) the cap changes nothing.  A negative tau keeps no key
   // in the reference, and no cap applies.
-  auto finish1 = [&](bool screened) {
+  static_assert(32 * RB == 64, "one wave row per lane");
+  auto set_thresholds = [&](float v, bool screened) {
     const float2 knm = a.knorm_max[kvh];
-    if (active) {
-      // complete the row max over the 32 lanes holding a row's keys, then the threshold
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          float v = mx[rb][i];
-          v = fmaxf(v, __shfl_xor(v, 1, 64));
-          v = fmaxf(v, __shfl_xor(v, 2, 64));
-          v = fmaxf(v, __shfl_xor(v, 4, 64));
-          v = fmaxf(v, __shfl_xor(v, 8, 64));
-          v = fmaxf(v, __shfl_xor(v, 16, 64));
-          const float m = v * a.sm_scale;   // fl(max * c) == max of fl(s * c) for c > 0
-          const int row = rb * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
-          const bool ok = wrow0 + row < a.N;   // padded rows never vote (exact_2.py:121)
-          float x0 = ok ? min_arg_for(m - tau, a.sm_scale) : INFINITY;
-          if (screened && ok && tau >= 0.0f) {
-            const float2 qn = a.qnorm[(int64_t)h * a.q_rows_pad + wrow0 + row];
-            const float delta = 1.001f * (qn.y * knm.y + 0x1p-15f * (qn.x + qn.y) * (knm.x + knm.y));
-            x0 = fminf(x0, v - delta);
-          }
-          mx[rb][i] = x0;
-          if constexpr (WM == 1) ref[rb][i] = m - tau;   // perquery.py:210; exact_2.py:130
-          if constexpr (WM == 2) ref[rb][i] = m;         // perquery.py:215; exact_2.py:135
-          if (a.row_max && (lane & 31) == 0 && ok) a.row_max[(int64_t)h * a.N + wrow0 + row] = m;
-        }
+    if (!active) return;
+    const int grow = wrow0 + lane;
+    const bool ok = grow < a.N;            // padded rows never vote (exact_2.py:121)
+    const float m = v * a.sm_scale;        // fl(max * c) == max of fl(s * c) for c > 0
+    float x0 = ok ? min_arg_for(m - tau, a.sm_scale) : INFINITY;
+    if (screened && ok && tau >= 0.0f) {
+      const float2 qn = a.qnorm[(int64_t)h * a.q_rows_pad + grow];
+      const float delta = 1.001f * (qn.y * knm.y + 0x1p-15f * (qn.x + qn.y) * (knm.x + knm.y));
+      x0 = fminf(x0, v - delta);
     }
+    if (a.row_max && ok) a.row_max[(int64_t)h * a.N + grow] = m;
+    const float rf = WM == 1 ? m - tau : m;   // perquery.py:210, 215; exact_2.py:130, 135
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int r0 = rb * 32 + (i >> 2) * 8 + (i & 3);     // the row of lanes 0-31; lanes 32-63: + 4
+        mx[rb][i] = row_value(x0, r0);
+        if constexpr (WM != 0) ref[rb][i] = row_value(rf, r0);
+      }
+  };
+  // three-product sweep: the row max over the 32 lanes holding a row's keys (mx: the raw dot's
+  // running max per row slot), into the row's lane
+  auto finish1 = [&]() {
+    float v = 0.0f;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        float x = mx[rb][i];
+        x = fmaxf(x, __shfl_xor(x, 1, 64));
+        x = fmaxf(x, __shfl_xor(x, 2, 64));
+        x = fmaxf(x, __shfl_xor(x, 4, 64));
+        x = fmaxf(x, __shfl_xor(x, 8, 64));
+        x = fmaxf(x, __shfl_xor(x, 16, 64));
+        const int r0 = rb * 32 + (i >> 2) * 8 + (i & 3);
+        const float lo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 0));
+        const float hi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 32));
+        v = lane == r0 ? lo : (lane == r0 + 4 ? hi : v);
+      }
+    set_thresholds(v, false);
   };
 
   auto run_pass = [&](auto passc) {
@@ -1270,7 +1291,7 @@ void score_kernel(ScoreArgs a) {
       chunk_end(c);
     }
     if (active && pendingB) flush(passc, accB, keyB);
-    if constexpr (pass == 0) finish1(false);
+    if constexpr (pass == 0) finish1();
   };
   if constexpr (MODE == 1) {
     // the screen: each row's exact raw maximum, or the workgroup's fallback flag
@@ -1290,7 +1311,6 @@ void score_kernel(ScoreArgs a) {
   } else {
     // pass 1: the screen's row maxima, or the three-product sweep where it fell back or is off
     // the screen's workgroups covering this one's rows (4 waves of 32 RB rows each)
-    bool exact1 = true;
     bool screen_ok = a.screened;
     {
       constexpr int SG = score_waves<false, 0, 1>() * 32 * RB;
@@ -1299,19 +1319,11 @@ void score_kernel(ScoreArgs a) {
         screen_ok = screen_ok && a.sflags[h * ng_s + gs] == 0;
     }
     if (screen_ok) {
-      exact1 = false;
-      if (active) {
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int row = wrow0 + rb * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
-            mx[rb][i] = row < rows_total ? a.srmax[(int64_t)h * a.q_rows_pad + row] : 0.0f;
-          }
-      }
+      const int row = wrow0 + lane;
+      set_thresholds(row < rows_total ? a.srmax[(int64_t)h * a.q_rows_pad + row] : 0.0f, true);
+    } else {
+      run_pass(std::integral_constant<int, 0>{});
     }
-    if (exact1) run_pass(std::integral_constant<int, 0>{});
-    else finish1(true);
     if constexpr (PQ == 6) {
       // thresholds only: every row's x0, replicated over the 32 lanes holding its keys
       if (active && (lane & 31) == 0) {

@@ -79,7 +79,7 @@ __global__ __launch_bounds__(512, 1) void score6_kernel(ScoreArgs a) {
   __shared__ u32x4 lds[NBUF][BUF_U];
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform: SGPR addresses
   const int rows_total = a.nt * T;
   const int ngroups = (rows_total + WG_ROWS - 1) / WG_ROWS;
   int h, g;
@@ -108,6 +108,34 @@ __global__ __launch_bounds__(512, 1) void score6_kernel(ScoreArgs a) {
   uint8_t* vrow = a.votes + ((int64_t)h * a.nt + wrow0 / T) * a.votes_stride;
   auto tile_ok = [&](int j) { return wrow0 + j * T < rows_total; };
 
+  // ---- keep thresholds x0 on the raw dot from the screen's exact row maxima.  For tau >= 0 the
+  // threshold is capped at max - delta (delta bounds the fp6 score's distance from the screen's
+  // exact dot, sta_fp6.h: fast6_delta), so a row's best key keeps its vote, as in the reference
+  // whose two passes share one dot.  Row block 0's accumulators start from -x0 (held in the
+  // AGPRs beside the Q operands), so its products accumulate s - x0 and the keep test is the
+  // accumulator's sign (that rounding, ~1e-6 of the score, is far inside the correction's error);
+  // row block 1 keeps x0 in VGPRs and subtracts it (the register file holds one set of each).
+  float* xs = (float*)&lds[NBUF - 1][0] + wave * 64;
+  {
+    // one row per lane, read back into the lane's 32 row slots (min_arg_for's division and
+    // nextafter steps on every slot cost each wave 32 times as many)
+    static_assert(32 * RB == 64, "one wave row per lane");
+    const float2 knm = a.knorm_max[kvh], kd = a.k6dmax[kvh];
+    const int row = wrow0 + lane;
+    const bool ok = active && row < a.N;       // padded rows never vote (exact_2.py:121)
+    const int64_t ri = (int64_t)h * a.q_rows_pad + (row < rows_total ? row : 0);
+    const float v = a.srmax[ri];
+    const float m = v * a.sm_scale;            // fl(max * c) == max of fl(s * c) for c > 0
+    float x = ok ? min_arg_for(m - tau, a.sm_scale) : INFINITY;
+    if (ok && tau >= 0.0f) {
+      const float2 qn = a.qnorm[ri], qd = a.q6dn[ri];
+      x = fminf(x, v - fast6_delta(qn.x, qn.y, qd.x, qd.y, knm.x, knm.y, kd.x, kd.y));
+    }
+    if (a.row_max && ok) a.row_max[(int64_t)h * a.N + row] = m;
+    // through the last chunk buffer, which no copy reaches before the sweep's first barrier
+    xs[lane] = -x;
+  }
+
   // ---- Q operands: bf16 hi fragments (AGPRs), fp6 units and their scale dwords ----
   const int64_t qrb0 = (int64_t)h * (a.q_rows_pad >> 5) + wrow0 / 32;
   u32x4 qhi[RB][S];
@@ -128,37 +156,24 @@ __global__ __launch_bounds__(512, 1) void score6_kernel(ScoreArgs a) {
     qsc[rb] = ok ? a.q6sc[(qrb0 + rb) * 64 + lane] : 0x7f7f7f7fu;
   }
 
-  // ---- keep thresholds x0 on the raw dot from the screen's exact row maxima.  For tau >= 0 the
-  // threshold is capped at max - delta (delta bounds the fp6 score's distance from the screen's
-  // exact dot, sta_fp6.h: fast6_delta), so a row's best key keeps its vote, as in the reference
-  // whose two passes share one dot.  Row block 0's accumulators start from -x0 (held in the
-  // AGPRs beside the Q operands), so its products accumulate s - x0 and the keep test is the
-  // accumulator's sign (that rounding, ~1e-6 of the score, is far inside the correction's error);
-  // row block 1 keeps x0 in VGPRs and subtracts it (the register file holds one set of each).
-  floatx16 nx0[RB];
-  {
-    const float2 knm = a.knorm_max[kvh], kd = a.k6dmax[kvh];
+  // -x0 of the lane's row slots, as scalars (a 16-register tuple that does not fit is spilled whole)
+  float nx0[RB][16];
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
+  for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int row = wrow0 + rb * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
-        const bool ok = active && row < a.N;   // padded rows never vote (exact_2.py:121)
-        const int64_t ri = (int64_t)h * a.q_rows_pad + (row < rows_total ? row : 0);
-        const float v = a.srmax[ri];
-        const float m = v * a.sm_scale;          // fl(max * c) == max of fl(s * c) for c > 0
-        float x = ok ? min_arg_for(m - tau, a.sm_scale) : INFINITY;
-        if (ok && tau >= 0.0f) {
-          const float2 qn = a.qnorm[ri], qd = a.q6dn[ri];
-          x = fminf(x, v - fast6_delta(qn.x, qn.y, qd.x, qd.y, knm.x, knm.y, kd.x, kd.y));
-        }
-        nx0[rb][i] = -x;
-        if (a.row_max && (lane & 31) == 0 && ok) a.row_max[(int64_t)h * a.N + row] = m;
-      }
-    asm volatile("" : "+a"(nx0[0]));
-  }
+    for (int i = 0; i < 16; ++i) {
+      nx0[rb][i] = xs[rb * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3)];
+      if (rb == 0) asm volatile("" : "+a"(nx0[rb][i]));
+    }
   // the accumulator's start and the kept test of row block rb
-  auto acc0 = [&](int rb) { return rb == 0 ? nx0[0] : floatx16{}; };
+  auto acc0 = [&](int rb) {
+    floatx16 x = {};
+    if (rb == 0) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x[i] = nx0[0][i];
+    }
+    return x;
+  };
   auto dropped = [&](float v, int rb, int i) {
     return (int)(__float_as_uint(rb == 0 ? v : v + nx0[rb][i]) >> 31);
   };
@@ -169,11 +184,10 @@ __global__ __launch_bounds__(512, 1) void score6_kernel(ScoreArgs a) {
   const u32x4* k6u = (const u32x4*)(a.k6 + (int64_t)kvh * (a.k_rows_pad >> 5) * NU * 192);
   const u32x4* k6s = (const u32x4*)(a.k6sc + (int64_t)kvh * (a.k_rows_pad >> 5) * 64);
   const uint32_t loff = (uint32_t)lane * 16u;
-  const int wave_s = __builtin_amdgcn_readfirstlane(wave);
   auto issue = [&](int c, u32x4* dst) {
 #pragma unroll
     for (int j = 0; j < CMAX; ++j) {
-      const int i = j * NW + wave_s;
+      const int i = j * NW + wave;
       if (i < NHI) {   // (32-key block, k step) i: its 1 KB of hi units, packed
         copy16_to_lds_s(khi + (int64_t)c * SBC * S * 128 + 128 * i, loff, lds_addr(dst + 64 * i));
       } else if (i < NHI + NF6) {
@@ -185,7 +199,7 @@ __global__ __launch_bounds__(512, 1) void score6_kernel(ScoreArgs a) {
   };
   // this wave's copies per chunk; wait until at most n chunks of them are in flight (vector
   // memory operations complete in order; vote stores in between only make the wait stricter)
-  const bool many = (NCP - wave_s + NW - 1) / NW == CMAX;
+  const bool many = (NCP - wave + NW - 1) / NW == CMAX;
   auto wait_copies = [&](int n) {
     constexpr int E = (7 << 4) | (15 << 8);   // expcnt / lgkmcnt: no wait
     constexpr int A1 = CMAX, A2 = 2 * CMAX, B1 = CMAX - 1, B2 = 2 * (CMAX - 1);
