@@ -75,6 +75,10 @@ struct ScoreArgs {
   int screened;           // set by the launcher: the screen kernel ran before the pass-2 kernel
   float* srmax;           // (H, q_rows_pad) the screen's exact raw row maxima
   int* sflags;            // (H, ngroups) the screen's fallback flags
+  int keys1;              // set by the launcher: pass 1 ran as the key-split sweep, and srmax holds
+                          // order keys (row_key) instead of floats; sflags is not written
+  int pieces, pchunks;    // set by the launcher, per launch: a row group's 64-key chunks are split
+                          // over `pieces` workgroups of at most `pchunks` chunks each
   float* xthr;            // thresholds-only instance: (H, q_rows_pad) each row's x0 (+inf: no row)
   // pass 2 with one bf16 product plus an fp6 correction (plain votes only, sta_score6.hip)
   int want_fast6;         // caller: the fragments carry the fp6 operands (16-bit inputs)
@@ -356,6 +360,37 @@ hipError_t launch_decode_select(const DecodeArgs& a, hipStream_t st);
 int decode_nsplit(int k_max);
 hipError_t launch_decode_attend(int dtype, int D, const DecodeArgs& a, hipStream_t st);
 
+// fp32 <-> unsigned with the same order (-0 folded into +0); no value but a NaN maps to 0, which the
+// rope pre-kernel leaves in srmax as "no maximum yet"
+__device__ __forceinline__ uint32_t row_key(float v) {
+  const uint32_t b = __float_as_uint(v + 0.0f);
+  return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+}
+__device__ __forceinline__ float row_key_value(uint32_t k) {
+  return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
+}
+// the raw maximum of fragment row i (of H * q_rows_pad) as pass 1 left it
+__device__ __forceinline__ float row_max_of(const ScoreArgs& a, int64_t i) {
+  return a.keys1 ? row_key_value(((const uint32_t*)a.srmax)[i]) : a.srmax[i];
+}
+
+// Workgroup `bid` of H heads x ngroups row groups x pieces key pieces.  XCD-aware: workgroup i runs
+// on XCD i % 8, so with H a multiple of 8 a head stays on one XCD; the heaviest groups come first.
+__device__ __forceinline__ void score_workgroup(int bid, int H, int ngroups, int pieces, int& h, int& g, int& piece) {
+  int rest;
+  if ((H & 7) == 0) {
+    const int hpx = H >> 3;
+    const int r = bid >> 3;
+    h = (bid & 7) * hpx + r % hpx;
+    rest = r / hpx;
+  } else {
+    h = bid % H;
+    rest = bid / H;
+  }
+  g = ngroups - 1 - rest / pieces;
+  piece = rest % pieces;
+}
+
 // Whether the fp6 pass-2 kernel (sta_score6.hip) serves workgroup g (wg_rows query rows) of
 // head h in the plain pass 2; the three-product kernel then skips it.  It does when the launcher
 // enabled it, the screened pass 1 resolved every row of the workgroup (its 256-row workgroups
@@ -366,8 +401,9 @@ __device__ inline bool fast6_serves(const ScoreArgs& a, int h, int g, int D, int
   const int rows_total = a.q_rows_pad;
   constexpr int SG = 256;
   const int ng_s = (rows_total + SG - 1) / SG;
-  for (int gs = g * wg_rows / SG; gs < min((g + 1) * wg_rows / SG, ng_s); ++gs)
-    if (a.sflags[h * ng_s + gs] != 0) return false;
+  if (!a.keys1)
+    for (int gs = g * wg_rows / SG; gs < min((g + 1) * wg_rows / SG, ng_s); ++gs)
+      if (a.sflags[h * ng_s + gs] != 0) return false;
   const int kvh = h / (a.H / a.Hkv);
   const float2 qn = a.qnorm_max[h], kn = a.knorm_max[kvh], qd = a.q6dmax[h], kd = a.k6dmax[kvh];
   const float sg = fast6_sigma(qn.x, qn.y, qd.x, qd.y, kn.x, kn.y, kd.x, kd.y, a.sm_scale, D);

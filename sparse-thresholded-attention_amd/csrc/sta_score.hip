@@ -19,6 +19,8 @@
 #include <float.h>
 #include <stdlib.h>
 
+#include <algorithm>
+
 #include <type_traits>
 
 namespace sta {
@@ -160,7 +162,8 @@ __global__ __launch_bounds__(256) void rope_frag_kernel(const void* __restrict__
                                                         const float* __restrict__ inv_freq,
                                                         u32x4* __restrict__ frag, float2* __restrict__ norms,
                                                         uint64_t* __restrict__ planes6, uint32_t* __restrict__ scales6,
-                                                        float2* __restrict__ dnorms6, float2* __restrict__ trig) {
+                                                        float2* __restrict__ dnorms6, float2* __restrict__ trig,
+                                                        uint32_t* __restrict__ rowkeys) {
 #pragma clang fp contract(off)
   constexpr int C2 = D / 16;                 // threads per row
   const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -244,7 +247,10 @@ __global__ __launch_bounds__(256) void rope_frag_kernel(const void* __restrict__
       sh += __shfl_xor(sh, o, 64);
       sl += __shfl_xor(sl, o, 64);
     }
-    if (c == 0) norms[(int64_t)head * rows_pad + row] = make_float2(sqrtf(sh), sqrtf(sl));
+    if (c == 0) {
+      norms[(int64_t)head * rows_pad + row] = make_float2(sqrtf(sh), sqrtf(sl));
+      rowkeys[(int64_t)head * rows_pad + row] = 0u;   // the key-split pass 1 merges its row maxima here
+    }
     if constexpr (W6) write_fp6<D>(o1, o2, hi1, hi2, c, row, head, rows_pad, lds6[threadIdx.x >> 6], planes6, scales6, dnorms6);
   }
 }
@@ -321,12 +327,16 @@ __global__ __launch_bounds__(1024) void norm_max_kernel(const float2* __restrict
 // MODE 1 runs only the screened pass 1 (hi products, half the registers and LDS of the full
 // kernel, two waves per SIMD) and leaves each row's exact maximum, or the workgroup's fallback
 // flag, for MODE 0, which runs pass 2 (and the three-product pass 1 where the screen fell back).
+// MODE 2 is the pass 1 of small calls: every score as the four products the screen takes for its
+// candidates (so the same maxima, bit for bit), the keys of a row group split over workgroups and
+// the rows' maxima merged by atomicMax.  The screen's candidate phase takes each wave 100 k cycles
+// however short its rows are, and one workgroup per 256 rows leaves most of the chip idle.
 // Waves per workgroup.  The screen: 4 (one per SIMD, two workgroups per CU).  Pass 2 with plain
 // votes: 8 (two per SIMD sharing each LDS chunk; each block's epilogue follows its own MFMAs and
 // the SIMD's other wave fills the gap).  Pass 2 with per-query bits, weighted votes or row counts
 // needs more registers: 4 waves, each overlapping a block's epilogue with the next block's MFMAs.
 template <bool RC, int PQ, int MODE>
-constexpr int score_waves() { return MODE == 1 ? 4 : ((PQ == 0 && !RC) ? 8 : 4); }
+constexpr int score_waves() { return MODE != 0 ? 4 : ((PQ == 0 && !RC) ? 8 : 4); }
 
 template <int D, int T, bool RC, int PQ, int RB, int MODE>
 __global__ __launch_bounds__((64 * score_waves<RC, PQ, MODE>()), (MODE == 1 ? 2 : 1))
@@ -372,19 +382,8 @@ void score_kernel(ScoreArgs a) {
   };
   const int rows_total = a.nt * T;               // == q_rows_pad
   const int ngroups = (rows_total + WG_ROWS - 1) / WG_ROWS;
-  int h, g;
-  {
-    const int bid = blockIdx.x;
-    if ((a.H & 7) == 0) {  // XCD-aware: workgroup i runs on XCD i % 8; keep a head on one XCD
-      const int hpx = a.H >> 3;
-      const int r = bid >> 3;
-      h = (bid & 7) * hpx + r % hpx;
-      g = ngroups - 1 - r / hpx;
-    } else {
-      h = bid % a.H;
-      g = ngroups - 1 - bid / a.H;
-    }
-  }
+  int h, g, piece;
+  score_workgroup(blockIdx.x, a.H, ngroups, MODE == 1 ? 1 : a.pieces, h, g, piece);
   // plain votes: the workgroups the fp6 pass-2 kernel served are done
   if constexpr (MODE == 0 && PLAIN) {
     if (fast6_serves(a, h, g, D, WG_ROWS)) return;
@@ -395,9 +394,14 @@ void score_kernel(ScoreArgs a) {
   const int hi_max = a.q_pos_base + min(g * WG_ROWS + WG_ROWS, rows_total);
   const int qpos0 = a.q_pos_base + wrow0;          // position of the wave's first row
   const int hi_w = qpos0 + 32 * RB;                // keys past the wave's last query are masked
-  const int nchunks = (hi_max + CK - 1) / CK;
+  // this workgroup's chunks: [c0, nchunks) (the screen takes whole rows)
+  const int c0 = MODE == 1 ? 0 : piece * a.pchunks;
+  const int nall = (hi_max + CK - 1) / CK;
+  const int nchunks = MODE == 1 ? nall : min(nall, c0 + a.pchunks);
+  if (c0 >= nchunks) return;
   // chunks entirely below N whose keys are causal for every query of the workgroup
-  const int nfull = min(min(nchunks, (a.q_pos_base + g * WG_ROWS + 1) / CK), a.N / CK);
+  const int nfull_all = min(min(nall, (a.q_pos_base + g * WG_ROWS + 1) / CK), a.N / CK);
+  const int nfull = min(nfull_all, nchunks);
   const float tau = a.tau[h];
   // the wave's tiles j = 0 .. NTW-1 start at row wrow0 + j T; one store instruction writes two
   // tiles' rows of a key (lanes 0-31 tile j, lanes 32-63 tile j + 1)
@@ -416,8 +420,8 @@ void score_kernel(ScoreArgs a) {
     for (int s = 0; s < S; ++s) {
       const int64_t u = (((int64_t)h * (a.q_rows_pad >> 5) + wrow0 / 32 + rb) * S + s) * 128 + lane;
       qhi[rb][s] = ok ? a.qfrag[u] : u32x4{0, 0, 0, 0};
-      if constexpr (MODE == 0) asm volatile("" : "+a"(qhi[rb][s]));
-      if constexpr (MODE == 0) {
+      if constexpr (MODE != 1) asm volatile("" : "+a"(qhi[rb][s]));
+      if constexpr (MODE != 1) {
         qlo[rb][s] = ok ? a.qfrag[u + 64] : u32x4{0, 0, 0, 0};
         asm volatile("" : "+a"(qlo[rb][s]));
       }
@@ -534,14 +538,27 @@ void score_kernel(ScoreArgs a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) { ref[rb][i] = 0.0f; rc[rb][i] = 0; }
 
-  // 32 keys x this wave's rows, one k step: hi.hi + hi.lo + lo.hi, small terms first
+  // 32 keys x this wave's rows, one k step: hi.hi + hi.lo + lo.hi, small terms first; MODE 2: the
+  // screen's four products in its order
+  constexpr int NPROD = MODE == 2 ? 4 : 3;
   auto mfma3 = [&](u32x4 bh, u32x4 bl, int s, floatx16* acc) {
+    if constexpr (MODE == 2) {
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) acc[rb] = mfma32(qlo[rb][s], bh, acc[rb]);
+      for (int rb = 0; rb < RB; ++rb) acc[rb] = mfma32(qhi[rb][s], bh, acc[rb]);
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) acc[rb] = mfma32(qhi[rb][s], bl, acc[rb]);
+      for (int rb = 0; rb < RB; ++rb) acc[rb] = mfma32(qhi[rb][s], bl, acc[rb]);
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) acc[rb] = mfma32(qhi[rb][s], bh, acc[rb]);
+      for (int rb = 0; rb < RB; ++rb) acc[rb] = mfma32(qlo[rb][s], bh, acc[rb]);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) acc[rb] = mfma32(qlo[rb][s], bl, acc[rb]);
+    } else {
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) acc[rb] = mfma32(qlo[rb][s], bh, acc[rb]);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) acc[rb] = mfma32(qhi[rb][s], bl, acc[rb]);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) acc[rb] = mfma32(qhi[rb][s], bh, acc[rb]);
+    }
   };
   auto ldb = [&](const u32x4* buf, int sb, int s, int hl) { return buf[(sb * S + s) * 128 + 64 * hl + lane]; };
   // Instruction schedule of one 32-key block (S k steps): the K fragments of step s + 1 are read
@@ -555,7 +572,7 @@ void score_kernel(ScoreArgs a) {
 #pragma unroll
     for (int s = 0; s < S; ++s) {
 #pragma unroll
-      for (int m = 0; m < 3 * RB; ++m) {
+      for (int m = 0; m < NPROD * RB; ++m) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);    // MFMA
         if (m == 0 && s >= 1 && s + 1 < S) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // step s + 1
         if constexpr (valu_per_mfma > 0) __builtin_amdgcn_sched_group_barrier(0x002, valu_per_mfma, 0);
@@ -1135,7 +1152,7 @@ void score_kernel(ScoreArgs a) {
     if (screened && ok && tau >= 0.0f) {
       const float2 qn = a.qnorm[(int64_t)h * a.q_rows_pad + grow];
       const float delta = 1.001f * (qn.y * knm.y + 0x1p-15f * (qn.x + qn.y) * (knm.x + knm.y));
-      x0 = fminf(x0, v - delta);
+      if (delta < INFINITY) x0 = fminf(x0, v - delta);   // no bound: rows or keys that are not finite
     }
     if (a.row_max && ok) a.row_max[(int64_t)h * a.N + grow] = m;
     const float rf = WM == 1 ? m - tau : m;   // perquery.py:210, 215; exact_2.py:130, 135
@@ -1148,9 +1165,9 @@ void score_kernel(ScoreArgs a) {
         if constexpr (WM != 0) ref[rb][i] = row_value(rf, r0);
       }
   };
-  // three-product sweep: the row max over the 32 lanes holding a row's keys (mx: the raw dot's
-  // running max per row slot), into the row's lane
-  auto finish1 = [&]() {
+  // after a pass-1 sweep: the row max over the 32 lanes holding a row's keys (mx: the raw dot's
+  // running max per row slot), in the row's lane
+  auto swept_max = [&]() {
     float v = 0.0f;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
@@ -1167,10 +1184,11 @@ void score_kernel(ScoreArgs a) {
         const float hi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 32));
         v = lane == r0 ? lo : (lane == r0 + 4 ? hi : v);
       }
-    set_thresholds(v, false);
+    return v;
   };
 
-  auto run_pass = [&](auto passc) {
+  // one sweep over the chunks [cb, ce)
+  auto run_pass = [&](auto passc, int cb, int ce) {
     constexpr int pass = decltype(passc)::value;
     constexpr std::integral_constant<bool, true> kPrev{};
     constexpr std::integral_constant<bool, false> kNoPrev{};
@@ -1183,22 +1201,23 @@ void score_kernel(ScoreArgs a) {
     // nothing the compiler tracks is in flight past this point: its own waits then stay out of
     // the sweep, whose copies it does not see
     __builtin_amdgcn_s_waitcnt(0);
-    for (int c = 0; c < NBUF - 1 && c < nchunks; ++c) issue(c, lds[c]);
-    wait_copies(min(nchunks, NBUF - 1) - 1);
+    for (int c = cb; c < cb + NBUF - 1 && c < ce; ++c) issue(c, lds[c % NBUF]);
+    wait_copies(min(ce - cb, NBUF - 1) - 1);
     __syncthreads();
+    const int nfl = min(nfull_all, ce);
     floatx16 accA[RB], accB[RB];
     bool pendingB = false;   // accB holds an unmasked block whose epilogue is still due
     int keyB = 0;
     // the buffer chunk c + NBUF - 1 lands in was last read in chunk c - 1, before the barrier
     auto chunk_begin = [&](int c) {
-      if (c + NBUF - 1 < nchunks) issue(c + NBUF - 1, lds[(c + NBUF - 1) % NBUF]);
+      if (c + NBUF - 1 < ce) issue(c + NBUF - 1, lds[(c + NBUF - 1) % NBUF]);
     };
     // chunk c + 1's copies have landed in LDS and every wave is done with chunk c
     auto chunk_end = [&](int c) {
-      if (c + 1 < nchunks) wait_copies(min(nchunks - 1, c + NBUF - 1) - (c + 1));
+      if (c + 1 < ce) wait_copies(min(ce - 1, c + NBUF - 1) - (c + 1));
       __syncthreads();
     };
-    int c = 0;
+    int c = cb;
     // the row-block pipeline (8-wave pass 2) over the fully causal chunks: pacc1 holds the
     // pending block's second row block, pdrop0 its first one's dropped-row count
     constexpr bool PIPE = !FUSED && PLAIN && pass == 1 && RB == 2;
@@ -1213,7 +1232,7 @@ void score_kernel(ScoreArgs a) {
         float w[RB] = {};
         store_key(pkey + (lane & 31), false, cnt, bm, w);
       };
-      for (; c < nfull; ++c) {
+      for (; c < nfl; ++c) {
         chunk_begin(c);
         const u32x4* buf = lds[c % NBUF];
         if (active) {
@@ -1221,7 +1240,7 @@ void score_kernel(ScoreArgs a) {
           for (int sb = 0; sb < SBC; ++sb) {
             int d1 = 0, d0 = 0;
             half_block(buf, sb, 0, pacc0, pacc1, RB - 1, d1);     // row block 0; previous block's 1
-            if (c > 0 || sb > 0) pipe_store(d1);
+            if (c > cb || sb > 0) pipe_store(d1);
             half_block(buf, sb, RB - 1, pacc1, pacc0, 0, d0);     // row block 1; this block's 0
             pdrop0 = d0;
             pkey = c * CK + sb * 32;
@@ -1229,19 +1248,19 @@ void score_kernel(ScoreArgs a) {
         }
         chunk_end(c);
       }
-      if (active && nfull > 0) {
+      if (active && nfl > cb) {
         int d1 = 0;
 #pragma unroll
         for (int i = 0; i < 16; ++i) d1 += (int)(__float_as_uint(pacc1[i] - mx[RB - 1][i]) >> 31);
         pipe_store(d1);
       }
     }
-    for (; c < nchunks; ++c) {
+    for (; c < ce; ++c) {
       chunk_begin(c);
       const u32x4* buf = lds[c % NBUF];
       if (active) {
-        if (FUSED && c < nfull) {
-          if (c == 0) fused_block(passc, kNoPrev, buf, 0, accA, accB, 0);
+        if (FUSED && c < nfl) {
+          if (c == cb) fused_block(passc, kNoPrev, buf, 0, accA, accB, 0);
           else fused_block(passc, kPrev, buf, 0, accA, accB, keyB);
           fused_block(passc, kPrev, buf, 1, accB, accA, c * CK);
           pendingB = true;
@@ -1291,7 +1310,6 @@ void score_kernel(ScoreArgs a) {
       chunk_end(c);
     }
     if (active && pendingB) flush(passc, accB, keyB);
-    if constexpr (pass == 0) finish1();
   };
   if constexpr (MODE == 1) {
     // the screen: each row's exact raw maximum, or the workgroup's fallback flag
@@ -1308,11 +1326,16 @@ void score_kernel(ScoreArgs a) {
         }
     }
     return;
+  } else if constexpr (MODE == 2) {
+    run_pass(std::integral_constant<int, 0>{}, c0, nchunks);
+    const float v = swept_max();
+    if (active && wrow0 + lane < rows_total)
+      atomicMax((uint32_t*)a.srmax + (int64_t)h * a.q_rows_pad + wrow0 + lane, row_key(v));
   } else {
     // pass 1: the screen's row maxima, or the three-product sweep where it fell back or is off
     // the screen's workgroups covering this one's rows (4 waves of 32 RB rows each)
     bool screen_ok = a.screened;
-    {
+    if (!a.keys1) {
       constexpr int SG = score_waves<false, 0, 1>() * 32 * RB;
       const int ng_s = (rows_total + SG - 1) / SG;
       for (int gs = g * WG_ROWS / SG; gs < min((g + 1) * WG_ROWS / SG, ng_s); ++gs)
@@ -1320,9 +1343,10 @@ void score_kernel(ScoreArgs a) {
     }
     if (screen_ok) {
       const int row = wrow0 + lane;
-      set_thresholds(row < rows_total ? a.srmax[(int64_t)h * a.q_rows_pad + row] : 0.0f, true);
+      set_thresholds(row < rows_total ? row_max_of(a, (int64_t)h * a.q_rows_pad + row) : 0.0f, true);
     } else {
-      run_pass(std::integral_constant<int, 0>{});
+      run_pass(std::integral_constant<int, 0>{}, 0, nall);
+      set_thresholds(swept_max(), false);
     }
     if constexpr (PQ == 6) {
       // thresholds only: every row's x0, replicated over the 32 lanes holding its keys
@@ -1337,7 +1361,7 @@ void score_kernel(ScoreArgs a) {
       }
       return;
     } else {
-      run_pass(std::integral_constant<int, 1>{});
+      run_pass(std::integral_constant<int, 1>{}, c0, nchunks);
     }
   }
 
@@ -1370,16 +1394,17 @@ static hipError_t launch_rope_frag_t(const void* x, int64_t hs, int64_t ts, int 
   const int64_t total = (int64_t)rows_pad * (D / 16);
   const int64_t blocks = (total + 255) / 256;
   float2* norms = frag_norms(frag, heads, rows_pad, D);
+  uint32_t* rowkeys = (uint32_t*)frag_rowmax(frag, heads, rows_pad, D);
   uint64_t* planes6 = want6 ? frag6_planes(frag, heads, rows_pad, D) : nullptr;
   uint32_t* scales6 = frag6_scales(frag, heads, rows_pad, D);
   float2* dn6 = frag6_dnorms(frag, heads, rows_pad, D);
   const dim3 grid((unsigned)blocks, (unsigned)((heads + ROPE_HG - 1) / ROPE_HG));
   if (want6)
     hipLaunchKernelGGL((rope_frag_kernel<DT, D, true>), grid, dim3(256), 0, st, x, hs, ts, heads, N,
-                       rows_pad, pos_base, pos_scale, rope_scale, inv_freq, frag, norms, planes6, scales6, dn6, trig);
+                       rows_pad, pos_base, pos_scale, rope_scale, inv_freq, frag, norms, planes6, scales6, dn6, trig, rowkeys);
   else
     hipLaunchKernelGGL((rope_frag_kernel<DT, D, false>), grid, dim3(256), 0, st, x, hs, ts, heads, N,
-                       rows_pad, pos_base, pos_scale, rope_scale, inv_freq, frag, norms, planes6, scales6, dn6, trig);
+                       rows_pad, pos_base, pos_scale, rope_scale, inv_freq, frag, norms, planes6, scales6, dn6, trig, rowkeys);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   // the row norms' maxima, and with the fp6 planes their rounding norms' in the same launch
@@ -1407,6 +1432,11 @@ static int exact_pass1_forced() {
   const char* e = getenv("STA_EXACT_PASS1");
   return e && e[0] == '1' ? 1 : 0;
 }
+// STA_SCREEN_PASS1=1: calls of every size run the screened pass 1, for comparisons
+static int screen_pass1_forced() {
+  const char* e = getenv("STA_SCREEN_PASS1");
+  return e && e[0] == '1' ? 1 : 0;
+}
 // STA_SCREEN_GATHER=1: the screen gathers its candidate keys from the K fragments even where the
 // (cos, sin) table is there, for comparisons
 static int screen_gather_forced() {
@@ -1416,6 +1446,52 @@ static int screen_gather_forced() {
 static int exact_pass2_forced() {
   const char* e = getenv("STA_EXACT_PASS2");
   return e && e[0] == '1' ? 1 : 0;
+}
+
+// How a launch splits its row groups' 64-key chunks over workgroups.
+struct ChunkSplit {
+  int pieces, chunks;    // workgroups per row group, chunks per workgroup
+};
+
+// chunks of row group g of wg_rows rows
+static int64_t group_chunks(int64_t q_pos_base, int64_t rows, int wg_rows, int g) {
+  return (q_pos_base + std::min<int64_t>((int64_t)(g + 1) * wg_rows, rows) + 63) / 64;
+}
+
+static int64_t chunk_steps(int H, int64_t q_pos_base, int64_t rows, int wg_rows) {
+  int64_t n = 0;
+  for (int g = 0; g < (rows + wg_rows - 1) / wg_rows; ++g) n += group_chunks(q_pos_base, rows, wg_rows, g);
+  return n * H;
+}
+
+// A CU holds one workgroup of pass 2 (or the key-split pass 1), so a grid of few row groups leaves
+// CUs idle and lasts as long as its longest group.  Time in chunk steps: a workgroup costs its
+// chunks plus `fixed` (Q fragments, thresholds, the copy pipeline's start); the unsplit grid,
+// heaviest first, the longer of its longest group and the average load; equal pieces something
+// between the average load and whole rounds.  The split has to win by a tenth.  Grids beyond two
+// workgroups per CU stay whole (28 heads x 4000 rows, PQ: 880 us whole, 901 us in pieces of 30
+// chunks).  Pass 2 split, calls on D 128: 8 heads x 9000 rows 758 -> 614 us, 32 x 3000 392 -> 366.
+static ChunkSplit split_chunks(int H, int64_t q_pos_base, int64_t rows, int wg_rows, int D, int waves) {
+  constexpr int CUS = 256;
+  const int ng = (int)((rows + wg_rows - 1) / wg_rows);
+  const int nall = (int)group_chunks(q_pos_base, rows, wg_rows, ng - 1);
+  ChunkSplit best{1, nall};
+  if ((int64_t)H * ng > 2 * CUS) return best;
+  const double fixed = (waves == 8 ? 6.0 : 10.0) * 128 / D;
+  const double load = (double)chunk_steps(H, q_pos_base, rows, wg_rows);
+  double t_best = 0.9 * std::max(nall + fixed, (load + fixed * H * ng) / CUS);
+  for (int c = 2; c < nall; c += (c + 1) / 2) {
+    int64_t wgs = 0;
+    for (int g = 0; g < ng; ++g) wgs += (group_chunks(q_pos_base, rows, wg_rows, g) + c - 1) / c;
+    wgs *= H;
+    const double rounds = (double)((wgs + CUS - 1) / CUS) * (c + fixed);
+    const double t = wgs <= CUS ? rounds : 0.5 * (rounds + (load + fixed * wgs) / CUS);
+    if (t < t_best) {
+      t_best = t;
+      best = ChunkSplit{(nall + c - 1) / c, c};
+    }
+  }
+  return best;
 }
 
 template <int D, int T, bool RC, int PQ>
@@ -1451,15 +1527,32 @@ static hipError_t launch_score_t(const ScoreArgs& a0, hipStream_t st) {
     a.k6sc = frag6_scales(a.kfrag, a.Hkv, a.k_rows_pad, D);
     a.k6dmax = frag6_dnorm_max(a.kfrag, a.Hkv, a.k_rows_pad, D);
   }
+  auto set_split = [&](const ChunkSplit& c) {
+    a.pieces = c.pieces;
+    a.pchunks = c.chunks;
+  };
   if (a.screened) {
-    // the screen is the same for every pass-2 epilogue: one instance per (D, T)
-    hipLaunchKernelGGL((score_kernel<D, T, false, 0, RB, 1>), dim3(a.H * ng_s), dim3(64 * WS), 0, st, a);
+    // Short calls take the key-split pass 1: up to 8192 (256-row group, 64-key chunk) steps, where
+    // the four products of every score cost what the screen's candidate phase does (32 heads:
+    // rows 2000 275 us a call against 294, 3000 399 against 391, 4500 760 against 646; 8 heads x
+    // 2048, D 64, fp32: 120 against 202).
+    a.keys1 = !screen_pass1_forced() && chunk_steps(a.H, a.q_pos_base, rows, 32 * RB * WS) <= 8192;
+    if (a.keys1) set_split(split_chunks(a.H, a.q_pos_base, rows, 32 * RB * WS, D, WS));
+    // the same for every pass-2 epilogue: one instance per (D, T)
+    if (a.keys1)
+      hipLaunchKernelGGL((score_kernel<D, T, false, 0, RB, 2>), dim3(a.H * ng_s * a.pieces), dim3(64 * WS), 0, st, a);
+    else
+      hipLaunchKernelGGL((score_kernel<D, T, false, 0, RB, 1>), dim3(a.H * ng_s), dim3(64 * WS), 0, st, a);
   }
+  // pass 2's keys are independent of each other, so any row group may be split (but its row counts)
+  a.pieces = 1;
+  a.pchunks = (int)(((int64_t)a.q_pos_base + rows + 63) / 64);
+  if (!RC && PQ != 6) set_split(split_chunks(a.H, a.q_pos_base, rows, 32 * RB * W2, D, W2));
   if (a.fast6) {
     const hipError_t e = launch_score6(D, T, a, st);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((score_kernel<D, T, RC, PQ, RB, 0>), dim3(a.H * ng_2), dim3(64 * W2), 0, st, a);
+  hipLaunchKernelGGL((score_kernel<D, T, RC, PQ, RB, 0>), dim3(a.H * ng_2 * a.pieces), dim3(64 * W2), 0, st, a);
   return hipGetLastError();
 }
 

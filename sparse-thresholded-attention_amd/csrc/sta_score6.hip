@@ -82,19 +82,8 @@ __global__ __launch_bounds__(512, 1) void score6_kernel(ScoreArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform: SGPR addresses
   const int rows_total = a.nt * T;
   const int ngroups = (rows_total + WG_ROWS - 1) / WG_ROWS;
-  int h, g;
-  {
-    const int bid = blockIdx.x;
-    if ((a.H & 7) == 0) {  // XCD-aware: workgroup i runs on XCD i % 8; keep a head on one XCD
-      const int hpx = a.H >> 3;
-      const int r = bid >> 3;
-      h = (bid & 7) * hpx + r % hpx;
-      g = ngroups - 1 - r / hpx;
-    } else {
-      h = bid % a.H;
-      g = ngroups - 1 - bid / a.H;
-    }
-  }
+  int h, g, piece;
+  score_workgroup(blockIdx.x, a.H, ngroups, a.pieces, h, g, piece);
   if (!fast6_serves(a, h, g, D, WG_ROWS)) return;   // the three-product kernel takes it
   const int kvh = h / (a.H / a.Hkv);
   const int wrow0 = g * WG_ROWS + wave * 32 * RB;
@@ -102,7 +91,9 @@ __global__ __launch_bounds__(512, 1) void score6_kernel(ScoreArgs a) {
   const int hi_max = a.q_pos_base + min(g * WG_ROWS + WG_ROWS, rows_total);
   const int qpos0 = a.q_pos_base + wrow0;
   const int hi_w = qpos0 + 32 * RB;
-  const int nchunks = (hi_max + CK - 1) / CK;
+  const int c0 = piece * a.pchunks;                // this workgroup's chunks: [c0, nchunks)
+  const int nchunks = min((hi_max + CK - 1) / CK, c0 + a.pchunks);
+  if (c0 >= nchunks) return;
   const int nfull = min(min(nchunks, (a.q_pos_base + g * WG_ROWS + 1) / CK), a.N / CK);
   const float tau = a.tau[h];
   uint8_t* vrow = a.votes + ((int64_t)h * a.nt + wrow0 / T) * a.votes_stride;
@@ -115,7 +106,7 @@ __global__ __launch_bounds__(512, 1) void score6_kernel(ScoreArgs a) {
   // AGPRs beside the Q operands), so its products accumulate s - x0 and the keep test is the
   // accumulator's sign (that rounding, ~1e-6 of the score, is far inside the correction's error);
   // row block 1 keeps x0 in VGPRs and subtracts it (the register file holds one set of each).
-  float* xs = (float*)&lds[NBUF - 1][0] + wave * 64;
+  float* xs = (float*)&lds[(c0 + NBUF - 1) % NBUF][0] + wave * 64;
   {
     // one row per lane, read back into the lane's 32 row slots (min_arg_for's division and
     // nextafter steps on every slot cost each wave 32 times as many)
@@ -124,7 +115,7 @@ __global__ __launch_bounds__(512, 1) void score6_kernel(ScoreArgs a) {
     const int row = wrow0 + lane;
     const bool ok = active && row < a.N;       // padded rows never vote (exact_2.py:121)
     const int64_t ri = (int64_t)h * a.q_rows_pad + (row < rows_total ? row : 0);
-    const float v = a.srmax[ri];
+    const float v = row_max_of(a, ri);
     const float m = v * a.sm_scale;            // fl(max * c) == max of fl(s * c) for c > 0
     float x = ok ? min_arg_for(m - tau, a.sm_scale) : INFINITY;
     if (ok && tau >= 0.0f) {
@@ -316,8 +307,8 @@ __global__ __launch_bounds__(512, 1) void score6_kernel(ScoreArgs a) {
 
   // ---- the sweep ----
   __builtin_amdgcn_s_waitcnt(0);   // nothing the compiler tracks stays in flight into the sweep
-  for (int c = 0; c < NBUF - 1 && c < nchunks; ++c) issue(c, lds[c]);
-  wait_copies(min(nchunks, NBUF - 1) - 1);
+  for (int c = c0; c < c0 + NBUF - 1 && c < nchunks; ++c) issue(c, lds[c % NBUF]);
+  wait_copies(min(nchunks - c0, NBUF - 1) - 1);
   __syncthreads();
   auto chunk_begin = [&](int c) {
     if (c + NBUF - 1 < nchunks) issue(c + NBUF - 1, lds[(c + NBUF - 1) % NBUF]);
@@ -329,18 +320,18 @@ __global__ __launch_bounds__(512, 1) void score6_kernel(ScoreArgs a) {
   constexpr std::integral_constant<bool, true> kPrev{};
   constexpr std::integral_constant<bool, false> kNoPrev{};
   floatx16 accA[RB], accB[RB];
-  int c = 0;
+  int c = c0;
   for (; c < nfull; ++c) {
     chunk_begin(c);
     const u32x4* buf = lds[c % NBUF];
     if (active) {
-      if (c == 0) block(kNoPrev, buf, 0, accA, accB, 0);
+      if (c == c0) block(kNoPrev, buf, 0, accA, accB, 0);
       else block(kPrev, buf, 0, accA, accB, c * CK - 32);
       block(kPrev, buf, 1, accB, accA, c * CK);
     }
     chunk_end(c);
   }
-  if (active && nfull > 0) flush(accB, nfull * CK - 32);
+  if (active && nfull > c0) flush(accB, nfull * CK - 32);
   for (; c < nchunks; ++c) {   // chunks on the diagonal or past N: masked, one block at a time
     chunk_begin(c);
     const u32x4* buf = lds[c % NBUF];
@@ -384,7 +375,7 @@ template <int D, int T>
 static hipError_t launch_score6_t(const ScoreArgs& a, hipStream_t st) {
   const int rows = a.nt * T;
   const int ng = (rows + 511) / 512;
-  hipLaunchKernelGGL((score6_kernel<D, T>), dim3(a.H * ng), dim3(512), 0, st, a);
+  hipLaunchKernelGGL((score6_kernel<D, T>), dim3(a.H * ng * a.pieces), dim3(512), 0, st, a);
   return hipGetLastError();
 }
 

@@ -1,0 +1,110 @@
+"""GPU: score passes whose keys are split over workgroups.
+
+Short calls take pass 1 as a sweep of every score in the screen's four products, each row group's
+keys split over workgroups and the row maxima merged; grids of few row groups split pass 2's keys.
+The maximum is over the same fp32 values and a key's votes need no other key, so both agree with
+the unsplit kernels bit for bit: with the screened pass 1 (STA_SCREEN_PASS1=1), and with the
+row-count instances of pass 2, which stay whole.
+"""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def say(msg):
+    print(f"[case] {msg}", flush=True)
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _need_gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    import _sta_native
+    _sta_native.lib()
+
+
+def _inputs(H, Hkv, N, D, dt, seed):
+    from synthetic import base_inv_freq, planted_inputs
+    q, k, v = planted_inputs(seed, H, Hkv, N, D, 0.01, dt, DEV)
+    return q, k, v, base_inv_freq(D, 10000.0).to(DEV), torch.full((H,), 4.0)
+
+
+CASES = [
+    # (H, Hkv, N, D, dtype, tile, q_pos_base): one short piece; the ends of 64-key chunks and of 256-
+    # and 512-row groups; phantom keys; head counts off the XCD map; the last call below the limit of
+    # 8192 (row group, chunk) steps and the first above; long rows of few heads (pass 2 split alone)
+    (1, 1, 1, 128, torch.bfloat16, 64, 0),
+    (2, 1, 65, 128, torch.bfloat16, 64, 0),
+    (3, 3, 257, 64, torch.float16, 32, 0),
+    (8, 8, 512, 128, torch.float32, 64, 0),
+    (5, 5, 513, 64, torch.bfloat16, 64, 0),
+    (4, 2, 1000, 128, torch.float16, 32, 37),
+    (28, 4, 700, 64, torch.bfloat16, 64, 640),
+    (8, 2, 2048, 64, torch.float32, 64, 0),
+    (8, 8, 5632, 128, torch.bfloat16, 64, 0),
+    (8, 8, 5900, 128, torch.bfloat16, 64, 0),
+    (2, 2, 9001, 128, torch.bfloat16, 32, 0),
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_row_max_and_votes_match_the_screen(case, monkeypatch):
+    import _sta_native as native
+    H, Hkv, N, D, dt, tile, qpb = case
+    say(f"key split: H={H} Hkv={Hkv} N={N} D={D} {dt} tile={tile} q_pos_base={qpb}")
+    q, k, _, invf, tau = _inputs(H, Hkv, N, D, dt, 31)
+    sm = 1.0 / math.sqrt(D)
+    got = {}
+    for screen in (False, True):
+        monkeypatch.setenv("STA_SCREEN_PASS1", "1" if screen else "0")
+        for score in ("freq", "expmass"):
+            r = native.select_vote(q, k, tau, invf, 0.5, 1.0, sm, tile, qpb, want_row_counts=False, select_score=score)
+            torch.cuda.synchronize()
+            got[screen, score] = [x.cpu().numpy() for x in r if x is not None]
+    for score in ("freq", "expmass"):
+        for a, b in zip(got[False, score], got[True, score]):
+            assert np.array_equal(a, b), f"{score}: {int((a != b).sum())} of {a.size} entries differ"
+
+
+@pytest.mark.parametrize("H,Hkv,N,D,dt", [(16, 4, 1500, 128, torch.bfloat16), (3, 3, 300, 64, torch.float32),
+                                          (8, 8, 4133, 64, torch.float16)])
+def test_split_bits_match_the_whole_row_instances(H, Hkv, N, D, dt):
+    """PQ pass 2 without row counts (split) against the row-count instance (whole)."""
+    import _sta_native as native
+    say(f"key split, per-query bits: H={H} N={N} D={D} {dt}")
+    q, k, v, invf, tau = _inputs(H, Hkv, N, D, dt, 37)
+    whole = native.pq_select_bits(q, k, tau, invf, 0.5, 1.0, 1.0 / math.sqrt(D))
+    part = native.PqPlan(q, k, v, tau, invf, invf, 0.5, 1.0, k_max=512, want_votes=True, want_row_max=True).run()
+    torch.cuda.synchronize()
+    for name in ("row_max", "votes", "bits", "wvotes"):
+        a, b = whole[name].cpu().numpy(), part[name].cpu().numpy()
+        assert np.array_equal(a, b), f"{name}: {int((a != b).sum())} of {a.size} entries differ"
+    rc = whole["row_counts"].cpu().numpy().sum()
+    assert int(part["votes"].sum()) == int(rc)
+
+
+def test_rows_and_keys_that_are_not_finite(monkeypatch):
+    """An infinite query row and a NaN key: no bound caps their head's thresholds, and every other
+    row keeps what the screen's fallback (three products a score, rounded apart by the lo.lo term:
+    1e-4 on the maxima, a vote in 1e4 at the threshold) keeps."""
+    import _sta_native as native
+    H, N, D = 3, 700, 128
+    q, k, _, invf, tau = _inputs(H, H, N, D, torch.bfloat16, 41)
+    q[0, 0, 100] = float("inf")
+    k[0, 1, 300, 5] = float("nan")
+    got = []
+    for screen in ("0", "1"):
+        monkeypatch.setenv("STA_SCREEN_PASS1", screen)
+        votes, _, rm = native.select_vote(q, k, tau, invf, 0.5, 1.0, 1.0 / math.sqrt(D), 64, want_row_counts=False)
+        torch.cuda.synchronize()
+        got.append((votes.cpu().numpy(), rm.cpu().numpy()))
+    (va, ma), (vb, mb) = got
+    fine = np.isfinite(mb)
+    assert np.array_equal(fine, np.isfinite(ma))
+    assert np.abs(ma[fine] - mb[fine]).max() < 1e-4
+    assert (va != vb).mean() < 1e-4

@@ -33,6 +33,12 @@ def _need_gpu():
     _sta_native.lib()
 
 
+@pytest.fixture(autouse=True)
+def _screen_at_every_size(monkeypatch):
+    """Short calls take the key-split pass 1 (tests/test_gpu_keysplit.py); here they run the screen."""
+    monkeypatch.setenv("STA_SCREEN_PASS1", "1")
+
+
 def _kernel_a(q, k, tau, invf, ps, rs, tile, q_pos_base, exact):
     import _sta_native as native
     old = os.environ.pop("STA_EXACT_PASS1", None)
