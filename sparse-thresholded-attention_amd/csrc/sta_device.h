@@ -10,6 +10,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace sta {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -349,6 +351,38 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   x = (int)max((uint32_t)x, (uint32_t)__builtin_amdgcn_mov_dpp(x, 0x140, 0xf, 0xf, false));   // row_mirror
   return max(max((uint32_t)__builtin_amdgcn_readlane(x, 0), (uint32_t)__builtin_amdgcn_readlane(x, 16)),
              max((uint32_t)__builtin_amdgcn_readlane(x, 32), (uint32_t)__builtin_amdgcn_readlane(x, 48)));
+}
+
+// Transpose of the 32x32 bit matrix held by each half wave, lane i's word its row i: bit i of the
+// result in lane j is bit j of lane i's word.  Five exchanges (lane ^ 16, 8, 4, 2, 1) by DPP moves
+// and a row swap, each followed by one byte permute or one rotate and one bit select.
+__device__ __forceinline__ uint32_t bit_transpose32(uint32_t x) {
+  const int lane = threadIdx.x & 63;
+  auto dpp = [](uint32_t v, auto c) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, decltype(c)::value, 0xf, 0xf, false);
+  };
+  auto rotr = [](uint32_t v, uint32_t n) { return __builtin_amdgcn_alignbit(v, v, n); };
+  auto sel = [](uint32_t m, uint32_t a, uint32_t b) { return (a & m) | (b & ~m); };
+  const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);    // rows 2k and 2k + 1
+  x = __builtin_amdgcn_perm(r[1], r[0], lane & 16 ? 0x07060302u : 0x05040100u);
+  x = __builtin_amdgcn_perm(dpp(x, std::integral_constant<int, 0x128>{}), x, lane & 8 ? 0x03070105u : 0x06020400u);  // row_ror:8
+  uint32_t y = dpp(dpp(x, std::integral_constant<int, 0x141>{}), std::integral_constant<int, 0x1b>{});  // i ^ 7 ^ 3
+  x = sel(lane & 4 ? 0xf0f0f0f0u : 0x0f0f0f0fu, x, rotr(y, lane & 4 ? 4u : 28u));
+  y = dpp(x, std::integral_constant<int, 0x4e>{});                        // quad_perm 2,3,0,1
+  x = sel(lane & 2 ? 0xccccccccu : 0x33333333u, x, rotr(y, lane & 2 ? 2u : 30u));
+  y = dpp(x, std::integral_constant<int, 0xb1>{});                        // quad_perm 1,0,3,2
+  x = sel(lane & 1 ? 0xaaaaaaaau : 0x55555555u, x, rotr(y, lane & 1 ? 1u : 31u));
+  return x;
+}
+
+// the max over each half wave's 32 lanes, in every lane of the half
+__device__ __forceinline__ int half_max(int x) {
+  x = max(x, __builtin_amdgcn_mov_dpp(x, 0xb1, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_mov_dpp(x, 0x4e, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_mov_dpp(x, 0x141, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_mov_dpp(x, 0x140, 0xf, 0xf, false));
+  const auto r = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)x, false, false);
+  return max((int)r[0], (int)r[1]);
 }
 
 __device__ __forceinline__ float wave_shfl_xor(float v, int m) { return __shfl_xor(v, m, 64); }

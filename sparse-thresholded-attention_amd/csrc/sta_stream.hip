@@ -29,6 +29,12 @@
 //
 // One workgroup = one head and G consecutive tiles (wave w owns tile g*G + w); each K~ / V block
 // is staged once in LDS (double-buffered, V transposed) and read by all G waves.
+//
+// VALU-bound: a (tile, 32-key block) issues about 360 vector instructions (132 of the query
+// rotation, 40 of its packing, 112 of the masked softmax) beside 16 products.  The keep words
+// (lane = key, bit = query) turn into each query's mask by a 32x32 bit transpose in registers, and
+// the output is rescaled only when a maximum grows by more than 2^8.  32 heads x 16384, D 128,
+// bf16: a call 11.0 -> 10.2 ms against one LDS shuffle per key and a rescale at every new maximum.
 #include "sta_device.h"
 #include "sta_kernels.h"
 
@@ -119,7 +125,7 @@ struct StreamCfg {
 };
 
 template <int DT, int D, int BN, int G, bool FUSED>
-__global__ __launch_bounds__(G * 64, 1) void stream_kernel(StreamArgs a) {
+__global__ __launch_bounds__(G * 64, !FUSED && DT != DT_F32 ? 2 : 1) void stream_kernel(StreamArgs a) {
 #pragma clang fp contract(off)
   using Cfg = StreamCfg<DT, D, BN, G, FUSED>;
   constexpr bool X3 = Cfg::X3;
@@ -291,14 +297,17 @@ __global__ __launch_bounds__(G * 64, 1) void stream_kernel(StreamArgs a) {
     }
   };
 
-  // ---- the tile's keep bits of one block: lane l < BN holds key start + l ----
+  // ---- the tile's keep bits of one block: lane l holds keys start + 32 sb + l % 32 (both half waves
+  //      the same words) ----
   const uint32_t* brow = FUSED ? nullptr : a.bits + ((int64_t)h * a.nt + (tile_ok ? t : 0)) * a.bits_stride;
   const int64_t loc_lo = (int64_t)t * 32 - a.n_local + 1, loc_hi = (int64_t)t * 32 + 31;   // :260-261
   const int rows_hi = min(32, N - t * 32);                        // rows < N
-  auto load_bits = [&](int b) -> uint32_t {
-    if constexpr (FUSED) return 0u;
-    const int j = b * BN + lane;
-    return (tile_ok && lane < BN && b >= 0 && j <= P_top) ? brow[j] : 0u;
+  auto load_bits = [&](int b, uint32_t* w) {
+#pragma unroll
+    for (int sb = 0; sb < NSB; ++sb) {
+      const int j = b * BN + sb * 32 + q;
+      w[sb] = !FUSED && tile_ok && b >= 0 && j <= P_top ? brow[j] : 0u;
+    }
   };
 
   floatx16 oacc[RBS];
@@ -306,6 +315,7 @@ __global__ __launch_bounds__(G * 64, 1) void stream_kernel(StreamArgs a) {
   for (int rb = 0; rb < RBS; ++rb) oacc[rb] = floatx16{};
   float mR = -INFINITY, l_i = 0.0f;   // running max of the raw dots, running sum
   const float c2 = a.sm_scale * 1.44269504088896341f;
+  const float lazy = 8.0f / c2;
   float d = 0.0f;                 // running base (:252)
   int kept_q = 0, n_used = 0;
 
@@ -313,7 +323,8 @@ __global__ __launch_bounds__(G * 64, 1) void stream_kernel(StreamArgs a) {
     load_block(nb_wg - 1);
     store_block(0);
   }
-  uint32_t bits_cur = load_bits(nb_wg - 1);
+  uint32_t bits_cur[NSB], bits_next[NSB];
+  load_bits(nb_wg - 1, bits_cur);
   __syncthreads();
 
   for (int it = 0; it < nb_wg; ++it) {
@@ -321,13 +332,14 @@ __global__ __launch_bounds__(G * 64, 1) void stream_kernel(StreamArgs a) {
     const int p = it & 1;
     const bool more = it + 1 < nb_wg;
     if (more) load_block(b - 1);
-    const uint32_t bits_next = load_bits(b - 1);
+    load_bits(b - 1, bits_next);
     if (tile_ok && b < nblk) {
       const int start = b * BN;
       const int hi_t = min(P_top, start + BN - 1);                  // :271
-      // this lane's mask bits: query q, keys 32 sb + (i/4)*8 + 4 hf + i%4
+      // this lane's mask bits, query q: bit mbit(i) is key 32 sb + (i/4)*8 + 4 hf + i%4
       uint32_t mbits[NSB];
-      int cnt = 0;
+      auto mbit = [](int i) { return FUSED ? i : (i >> 2) * 8 + (i & 3); };
+      int c_q = 0;                                                  // keys of query q (:288)
       if constexpr (FUSED) {
         // S_a^T = K_a . Q_a^T (key rows, query columns), hi.lo terms first as in the score
         // kernel's pass 2; keep = s >= x0 (rows < N through x0 = +inf), causal, or forced (:285-286)
@@ -357,7 +369,7 @@ __global__ __launch_bounds__(G * 64, 1) void stream_kernel(StreamArgs a) {
             fb |= (uint32_t)(causal && forced) << i;
           }
           mbits[sb] = tb | fb;
-          cnt += __popc(mbits[sb]);
+          c_q += __popc(mbits[sb]);
           if (a.bits_out) {
             // the threshold bits as the score kernel lays them out: one word per key, bit = row
 #pragma unroll
@@ -371,44 +383,29 @@ __global__ __launch_bounds__(G * 64, 1) void stream_kernel(StreamArgs a) {
           }
         }
       } else {
-        // keep word of key start + lane: threshold bits, or every causal row when forced
-        uint32_t kw = 0;
-        {
-          const int j = start + lane;
-          if (lane < BN && j <= P_top) {
-            kw = bits_cur;
-            const bool forced = j < a.n_global || (j >= loc_lo && j <= loc_hi);   // :284
-            if (forced) {
-              const int lo_r = max(0, j - t * 32);                  // causal: qpos_i >= j
-              const uint32_t hi_mask = rows_hi >= 32 ? 0xffffffffu : ((1u << rows_hi) - 1u);
-              kw |= hi_mask & ~((1u << lo_r) - 1u);
-            }
-          }
-        }
+        // keep words (threshold bits, or every causal row when forced), transposed so that lane q
+        // holds query q's keys
 #pragma unroll
         for (int sb = 0; sb < NSB; ++sb) {
-          mbits[sb] = 0;
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int key = sb * 32 + (i >> 2) * 8 + 4 * hf + (i & 3);
-            const uint32_t w = (uint32_t)__shfl((int)kw, key, 64);
-            mbits[sb] |= ((w >> q) & 1u) << i;
+          const int j = start + sb * 32 + q;
+          uint32_t kw = bits_cur[sb];                               // 0 past P_top
+          const bool forced = j < a.n_global || (j >= loc_lo && j <= loc_hi);   // :284
+          if (forced && j <= P_top) {
+            const int lo_r = max(0, j - t * 32);                    // causal: qpos_i >= j
+            const uint32_t hi_mask = rows_hi >= 32 ? 0xffffffffu : ((1u << rows_hi) - 1u);
+            kw |= hi_mask & ~((1u << lo_r) - 1u);
           }
-          cnt += __popc(mbits[sb]);
+          const uint32_t tq = bit_transpose32(kw);
+          c_q += __popc(tq);
+          mbits[sb] = tq >> (4 * hf);
         }
       }
-      const int c_q = cnt + __shfl_xor(cnt, 32, 64);               // keys of query q (:288)
+      if constexpr (FUSED) c_q += __shfl_xor(c_q, 32, 64);
       int adv_i;
       if (a.adv_full) {
         adv_i = hi_t - start + 1;                                  // :303-304
       } else {
-        int m = c_q;                                               // :305-306
-        m = max(m, __shfl_xor(m, 1, 64));
-        m = max(m, __shfl_xor(m, 2, 64));
-        m = max(m, __shfl_xor(m, 4, 64));
-        m = max(m, __shfl_xor(m, 8, 64));
-        m = max(m, __shfl_xor(m, 16, 64));
-        adv_i = m;
+        adv_i = __builtin_amdgcn_readfirstlane(half_max(c_q));     // :305-306; both halves alike
       }
       if (!(a.use_skip && adv_i <= 0)) {                            // :319-322
         // ---- rotate the tile's queries by w = d + hi_t (one sin/cos per frequency) ----
@@ -485,12 +482,16 @@ __global__ __launch_bounds__(G * 64, 1) void stream_kernel(StreamArgs a) {
         for (int sb = 0; sb < NSB; ++sb)
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
-            const float v = ((mbits[sb] >> i) & 1u) ? sacc[sb][i] : -INFINITY;
+            // the score, or -inf: one bit field extract (0 or ~0) and one bit select
+            const uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)mbits[sb], (uint32_t)mbit(i), 1u);
+            const float v = __uint_as_float((__float_as_uint(sacc[sb][i]) & m) | (0xff800000u & ~m));
             sacc[sb][i] = v;
             bmax = fmaxf(bmax, v);
           }
         bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
-        const float mnew = fmaxf(mR, bmax);
+        // raised only by more than 2^8 (weights stay below 2^8, their relative rounding the same): some
+        // query of a tile meets a new maximum in most blocks, and each raise rescales the output
+        const float mnew = bmax > mR + lazy ? bmax : mR;
         const float msafe = (mnew == -INFINITY) ? 0.0f : mnew;
         const float alpha = __builtin_amdgcn_exp2f((mR - msafe) * c2);
         const float moff = -msafe * c2;
@@ -550,7 +551,8 @@ __global__ __launch_bounds__(G * 64, 1) void stream_kernel(StreamArgs a) {
         n_used += 1;
       }
     }
-    bits_cur = bits_next;
+#pragma unroll
+    for (int sb = 0; sb < NSB; ++sb) bits_cur[sb] = bits_next[sb];
     if (more) store_block(p ^ 1);
     __syncthreads();
   }
@@ -612,7 +614,13 @@ hipError_t launch_abs_rope(int dtype, int D, const void* x, int64_t hs, int64_t 
   return hipErrorInvalidValue;
 }
 
-constexpr int kStreamTiles = 8;        // tiles (waves) per workgroup, unfused sweep
+// Tiles (waves) per workgroup, unfused sweep.  A CU holds eight waves, two to a SIMD, by registers:
+// two workgroups of four tiles wait for each other's barriers less and leave less of a short call's
+// last round idle (16 heads x 12000, D 128, fp16: 3.01 ms against 3.23 with eight tiles; 32 x 16384
+// bf16: 10.0 either way).  fp32 stages twice the bytes a block, so long grids share each block among
+// eight tiles (32 heads x 4000, D 64: 670 us against 732; 8 heads x 4000, D 128: 811 against 731).
+constexpr int kStreamTiles = 4, kStreamTilesF32 = 8;
+constexpr int kStreamLongGrid = 2048;  // fp32: (head, tile) pairs, one wave each, that fill the chip
 constexpr int kStreamTilesFused = 4;   // fused sweep: one wave per SIMD, the register room the
                                        // selection fragments need
 
@@ -634,7 +642,7 @@ constexpr size_t stream_lds_t(bool fused) {
   if constexpr (stream_fused<DT, D, BN>()) {
     if (fused) return StreamCfg<DT, D, BN, kStreamTilesFused, true>::lds_bytes;
   }
-  return StreamCfg<DT, D, BN, kStreamTiles, false>::lds_bytes;
+  return StreamCfg<DT, D, BN, DT == DT_F32 ? kStreamTilesF32 : kStreamTiles, false>::lds_bytes;
 }
 
 size_t stream_lds_bytes(int dtype, int D, int BN, bool fused) {
@@ -664,6 +672,9 @@ static hipError_t launch_stream_t(const StreamArgs& a, hipStream_t st) {
     if (a.qfrag) return launch_stream_g<DT, D, BN, kStreamTilesFused, true>(a, st);
   }
   if (!a.bits) return hipErrorInvalidValue;
+  if constexpr (DT == DT_F32) {
+    if ((int64_t)a.H * a.nt > kStreamLongGrid) return launch_stream_g<DT, D, BN, kStreamTilesF32, false>(a, st);
+  }
   return launch_stream_g<DT, D, BN, kStreamTiles, false>(a, st);
 }
 

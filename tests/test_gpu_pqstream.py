@@ -354,3 +354,30 @@ def test_pqs_decode_rejects_bad_block_n():
         with pytest.raises(RuntimeError):
             native.DecodePlan(q, k, None, torch.ones(2), torch.ones(32), 199, k_max=1024, rule="stream",
                               block_n=bn).build_sets(torch.zeros(2, 1, 200, device=DEV))
+
+
+@pytest.mark.parametrize("dt,H,N,D,block_n", [(torch.float32, 2, 1283, 64, 64), (torch.float32, 24, 2780, 64, 32),
+                                              (torch.float16, 3, 257, 128, 64), (torch.bfloat16, 8, 33, 64, 32)])
+def test_stream_workgroup_sizes_and_mask_edges(dt, H, N, D, block_n):
+    """Both workgroup sizes of the fp32 sweep (24 heads x 87 tiles and more take eight tiles), the
+    bit-transposed masks at 32- and 64-key blocks, and tiles and blocks cut by the last row."""
+    import _sta_native as native
+    from synthetic import base_inv_freq, planted_inputs
+    say(f"stream masks: H={H} N={N} D={D} block_n={block_n} {dt}")
+    q, k, v = planted_inputs(61, H, H, N, D, 0.02, dt, DEV)
+    invf = base_inv_freq(D, 10000.0)
+    tau = torch.full((H,), 2.0)
+    r = native.pqstream_attention(q, k, v, tau, invf, invf, 0.5, 1.0, block_n=block_n, want_bits=True, fused="unfused")
+    torch.cuda.synchronize()
+    for h in range(0, H, 7):                                 # a few heads through the oracle
+        qn, odt = np_of(q[0, h:h + 1])
+        kn, _ = np_of(k[0, h:h + 1])
+        vn, _ = np_of(v[0, h:h + 1])
+        out, span, kept, _, _, _ = orc.pqstream(qn, kn, vn, odt, np.full(1, 2.0, np.float32), invf.numpy(), invf.numpy(),
+                                                0.5, 1.0, block_n=block_n, bits_in=r["bits"][h:h + 1].cpu().numpy(),
+                                                want_band=False)
+        assert np.array_equal(r["kept"][h:h + 1].cpu().numpy(), kept)
+        assert np.array_equal(r["span"][h:h + 1].cpu().numpy(), span)
+        err = np.abs(r["out"][h:h + 1].float().cpu().numpy() - out)
+        tol = 1e-4 if dt == torch.float32 else 2e-2 + 1e-2 * np.abs(out)
+        assert np.all(err <= tol), f"head {h}: {err.max():.3e}"
