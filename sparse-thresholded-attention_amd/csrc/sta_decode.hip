@@ -5,7 +5,7 @@
 //
 //   decode_qrot_kernel    the query rotated at fl(float(q_pos) * pos_scale)        (exact_2.py:250-257)
 //   decode_score_kernel   per-key scores under the selection geometry            (exact_2.py:235-271)
-//                         64 keys x up to 4 kv heads per workgroup: the key rotation's
+//                         64 keys x several kv heads per workgroup: the key rotation's
 //                         sin / cos is computed once per (key, frequency) and shared by the heads;
 //                         the query rows are rotated in the workgroup's LDS (decode_qrot_kernel
 //                         precomputes them when they outgrow it)
@@ -107,47 +107,70 @@ __global__ __launch_bounds__(D / 2) void decode_qrot_kernel(DecodeArgs a, float*
 }
 
 // ------------------------------------------------------------------------------------------
-// per-key scores (H, Q, M): 64 keys x HG kv heads per workgroup, 4 lanes per key.  Every head's
-// key rows are requested first (kept packed in registers), then the workgroup rotates its query
-// rows into LDS and computes the keys' sin / cos -- once per (key, frequency), shared by the
-// heads -- while the rows are in flight.
+// per-key scores (H, Q, M): 64 keys x hgt kv heads per workgroup, 4 lanes per key.  The key rows of
+// two heads are requested (kept packed in registers) while the two before are scored; the first
+// pair is in flight while the workgroup rotates its query rows into LDS and computes the keys'
+// sin / cos -- once per (key, frequency), shared by all the workgroup's heads: 16 accurate sincosf a
+// lane cost as much as scoring five heads, so more heads a workgroup save arithmetic and fewer
+// fill the chip (score_heads below).
 // ------------------------------------------------------------------------------------------
 constexpr int DEC_QLDS = 32 * 1024;           // LDS for rotated query rows
 
-template <int DT>
-constexpr int dec_hg() { return 4; }   // 4 kv heads: ~140 VGPRs, 3 waves per SIMD (8 heads: 2)
-
-// kv heads of one score workgroup and whether its rotated query rows fit its LDS
-int decode_score_hg(int dtype) { return dtype == DT_F32 ? dec_hg<DT_F32>() : dec_hg<DT_BF16>(); }
-bool decode_qrot_in_lds(int dtype, int H, int Hkv, int Q, int D) {
-  return (size_t)decode_score_hg(dtype) * (H / Hkv) * Q * D * 4 <= DEC_QLDS;
+// kv heads of one score workgroup, and whether their rotated query rows fit its LDS.  Time in units
+// of scoring one kv head for one query, fitted to the sweeps below: a workgroup costs 5 (sincos and
+// start) plus 0.7 + 0.3 per query row for each head, the grid its average load per CU plus 1.2
+// workgroups (the last round).  Calls, us, by heads per workgroup: 32 kv heads x 12288 keys 4: 48.9,
+// 8: 47.0, 16: 48.2, 32: 56.5; 32 x 40000 4: 243.8, 16: 236.5; 8 kv heads with 4 query heads each x
+// 32768 2: 65.1, 4: 63.5, 8: 60.7; 4 with 7 each x 20000 1: 45.9, 2: 43.9, 4: 48.1.
+static int score_heads(int H, int Hkv, int Q, int D, int M, bool& in_lds) {
+  const int rows = H / Hkv * Q;                // query rows per kv head
+  const size_t row_bytes = (size_t)rows * D * 4;
+  in_lds = row_bytes <= DEC_QLDS;
+  int best = 1;
+  double t_best = 0.0;
+  for (int g = 1; g < 2 * Hkv && g <= 32; g *= 2) {
+    if (g > 1 && in_lds && row_bytes * g > DEC_QLDS) break;
+    const int64_t wgs = (int64_t)((M + 63) / 64) * ((Hkv + g - 1) / g);
+    const double t = ((double)wgs / 256 + 1.2) * (5.0 + g * (0.7 + 0.3 * rows));
+    if (g == 1 || t < t_best) {
+      t_best = t;
+      best = g;
+    }
+  }
+  return best;
 }
 
 template <int DT, int D, bool QLDS>
-__global__ __launch_bounds__(256) void decode_score_kernel(DecodeArgs a) {
+__global__ __launch_bounds__(256) void decode_score_kernel(DecodeArgs a, int hgt) {
 #pragma clang fp contract(off)
-  constexpr int HG = dec_hg<DT>();
   constexpr int NP = D / 8;                   // rotation pairs per lane
   constexpr int ES = DT == DT_F32 ? 4 : 2;
   constexpr int UH = NP * ES / 16;            // 16-byte units per half row per lane
-  __shared__ __align__(16) float qs[QLDS ? DEC_QLDS / 4 : 1];
+  constexpr int E = 16 / ES;                  // elements per unit
+  // pair p of lane t: frequency fq(p), so that the 4 lanes of a key read 64 contiguous bytes a load
   const int t = threadIdx.x & 3;
+  auto fq = [&](int p) { return p / E * 4 * E + t * E + p % E; };
+  __shared__ __align__(16) float qs[QLDS ? DEC_QLDS / 4 : 1];
   const int j = blockIdx.x * 64 + (threadIdx.x >> 2);
   const int jc = j < a.M ? j : a.M - 1;
-  const int hk0 = blockIdx.y * HG;
-  const int nh = min(HG, a.Hkv - hk0);        // kv heads of this workgroup
+  const int hk0 = blockIdx.y * hgt;
+  const int nh = min(hgt, a.Hkv - hk0);       // kv heads of this workgroup
   const int G = a.H / a.Hkv;
-  u32x4 raw[HG][2 * UH];
+  u32x4 rawA[2][2 * UH], rawB[2][2 * UH];
+  // the key rows of heads hk0 + g and hk0 + g + 1; heads past the workgroup's reload its last row
+  auto load_pair = [&](int g, u32x4 (&raw)[2][2 * UH]) {
 #pragma unroll
-  for (int g = 0; g < HG; ++g) {
-    const int hk = hk0 + min(g, nh - 1);       // heads past Hkv reload a valid row, store nothing
-    const char* row = (const char*)a.k + ((int64_t)hk * a.k_hs + (int64_t)jc * a.k_ts + t * NP) * ES;
+    for (int e = 0; e < 2; ++e) {
+      const int hk = hk0 + min(g + e, nh - 1);
+      const char* row = (const char*)a.k + ((int64_t)hk * a.k_hs + (int64_t)jc * a.k_ts + t * E) * ES;
 #pragma unroll
-    for (int u = 0; u < UH; ++u) {
-      raw[g][u] = *(const u32x4*)(row + 16 * u);
-      raw[g][UH + u] = *(const u32x4*)(row + (D / 2) * ES + 16 * u);
+      for (int u = 0; u < UH; ++u) {
+        raw[e][u] = *(const u32x4*)(row + 64 * u);
+        raw[e][UH + u] = *(const u32x4*)(row + (D / 2) * ES + 64 * u);
+      }
     }
-  }
+  };
+  load_pair(0, rawA);
   const int R = nh * G * a.Q;                  // query rows: (kv head, q head of its group, query)
   if constexpr (QLDS) {
     // rotated at fl(float(q_pos0 + i) * pos_scale) (exact_2.py:250-257)
@@ -167,13 +190,13 @@ __global__ __launch_bounds__(256) void decode_score_kernel(DecodeArgs a) {
       qs[r * D + D / 2 + f] = p3 + p4;
     }
   }
-  // cos / sin of this key's frequencies t*NP .. t*NP + NP - 1
+  // cos / sin of this key's frequencies fq(0) .. fq(NP - 1)
   float cs[NP], sn[NP];
   {
     const float kb = (float)j * a.pos_scale_a;                            // exact_2.py:264
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
-      const float ang = kb * a.inv_freq_a[t * NP + p];
+      const float ang = kb * a.inv_freq_a[fq(p)];
       sincosf(ang, &sn[p], &cs[p]);
       cs[p] = cs[p] * a.rope_scale_a;
       sn[p] = sn[p] * a.rope_scale_a;
@@ -181,18 +204,16 @@ __global__ __launch_bounds__(256) void decode_score_kernel(DecodeArgs a) {
   }
   if constexpr (QLDS) __syncthreads();
   const float* qsrc = QLDS ? qs : a.qrot + (int64_t)hk0 * G * a.Q * D;
-#pragma unroll
-  for (int g = 0; g < HG; ++g) {
-    if (g >= nh) break;
+  auto score_head = [&](int g, const u32x4 (&raw)[2 * UH]) {
     float k1[NP], k2[NP];
 #pragma unroll
     for (int p = 0; p < NP; ++p) {                                        // exact_2.py:266-267
       float x1, x2;
       if constexpr (DT == DT_F32) {
-        x1 = __uint_as_float(raw[g][p / 4][p % 4]);
-        x2 = __uint_as_float(raw[g][UH + p / 4][p % 4]);
+        x1 = __uint_as_float(raw[p / 4][p % 4]);
+        x2 = __uint_as_float(raw[UH + p / 4][p % 4]);
       } else {
-        const uint32_t w1 = raw[g][p / 8][(p % 8) / 2], w2 = raw[g][UH + p / 8][(p % 8) / 2];
+        const uint32_t w1 = raw[p / 8][(p % 8) / 2], w2 = raw[UH + p / 8][(p % 8) / 2];
         const uint32_t h1 = (p & 1) ? (w1 >> 16) : (w1 & 0xffffu), h2 = (p & 1) ? (w2 >> 16) : (w2 & 0xffffu);
         x1 = DT == DT_BF16 ? __uint_as_float(h1 << 16) : f16_bits_to_f32(h1);
         x2 = DT == DT_BF16 ? __uint_as_float(h2 << 16) : f16_bits_to_f32(h2);
@@ -206,8 +227,8 @@ __global__ __launch_bounds__(256) void decode_score_kernel(DecodeArgs a) {
       float acc = 0.0f;
 #pragma unroll
       for (int p = 0; p < NP; p += 4) {
-        const float4 u = *(const float4*)(qr + t * NP + p);
-        const float4 w = *(const float4*)(qr + D / 2 + t * NP + p);
+        const float4 u = *(const float4*)(qr + fq(p));
+        const float4 w = *(const float4*)(qr + D / 2 + fq(p));
         acc = fmaf(u.x, k1[p], acc);
         acc = fmaf(w.x, k2[p], acc);
         acc = fmaf(u.y, k1[p + 1], acc);
@@ -223,6 +244,17 @@ __global__ __launch_bounds__(256) void decode_score_kernel(DecodeArgs a) {
       const int m = a.M - (a.Q - 1 - i);
       if (t == 0 && j < m) a.scores[((int64_t)hq * a.Q + i) * a.M + j] = acc * a.sm_scale;   // :270
     }
+  };
+  auto score_pair = [&](int g, const u32x4 (&raw)[2][2 * UH]) {
+    score_head(g, raw[0]);
+    if (g + 1 < nh) score_head(g + 1, raw[1]);
+  };
+  for (int g = 0; g < nh; g += 4) {
+    if (g + 2 < nh) load_pair(g + 2, rawB);
+    score_pair(g, rawA);
+    if (g + 2 >= nh) break;
+    if (g + 4 < nh) load_pair(g + 4, rawA);
+    score_pair(g + 2, rawB);
   }
 }
 
@@ -2046,13 +2078,15 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(DecodeArgs a, int n
 template <int DT, int D>
 static hipError_t launch_scores_t(const DecodeArgs& a0, float* qrot, hipStream_t st) {
   DecodeArgs a = a0;
-  dim3 grid((a.M + 63) / 64, (a.Hkv + dec_hg<DT>() - 1) / dec_hg<DT>());
-  if (decode_qrot_in_lds(DT, a.H, a.Hkv, a.Q, D)) {
-    hipLaunchKernelGGL((decode_score_kernel<DT, D, true>), grid, dim3(256), 0, st, a);
+  bool in_lds;
+  const int hgt = score_heads(a.H, a.Hkv, a.Q, D, a.M, in_lds);
+  const dim3 grid((a.M + 63) / 64, (a.Hkv + hgt - 1) / hgt);
+  if (in_lds) {
+    hipLaunchKernelGGL((decode_score_kernel<DT, D, true>), grid, dim3(256), 0, st, a, hgt);
   } else {
     hipLaunchKernelGGL((decode_qrot_kernel<DT, D>), dim3(a.H * a.Q), dim3(D / 2), 0, st, a, qrot);
     a.qrot = qrot;
-    hipLaunchKernelGGL((decode_score_kernel<DT, D, false>), grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL((decode_score_kernel<DT, D, false>), grid, dim3(256), 0, st, a, hgt);
   }
   return hipGetLastError();
 }

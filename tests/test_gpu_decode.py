@@ -317,3 +317,47 @@ def test_decode_tiled_scores_match_row_major(case):
     for name in names:
         assert torch.equal(tiled[name], rows[name]), name
     assert int((tiled["set_size"] > 0).sum()) == H * Q
+
+
+@pytest.mark.parametrize("case", [
+    # (H, Hkv, Q, M, D, dtype): one head a workgroup and a lone pair's first head; an odd head count
+    # over several pairs; heads past a workgroup's last; query rows that outgrow its LDS beside one,
+    # two and no kv head; long rows of many heads
+    (1, 1, 1, 1, 128, torch.bfloat16),
+    (3, 3, 1, 65, 64, torch.float16),
+    (7, 7, 1, 40000, 128, torch.bfloat16),
+    (20, 5, 1, 9000, 64, torch.float32),
+    (12, 12, 2, 20001, 128, torch.float32),
+    (8, 2, 15, 3000, 128, torch.bfloat16),
+    (28, 4, 1, 20000, 128, torch.float16),
+    (16, 1, 8, 700, 128, torch.bfloat16),
+])
+def test_decode_scores_over_heads_per_workgroup(case):
+    """The scores of every head against float64 of the same fp32 angles, within fp32 rounding of the
+    rotated rows (D products of magnitude |q||k| / D, 2^-22 each)."""
+    import _sta_native as native
+    from synthetic import base_inv_freq
+    H, Hkv, Q, M, D, dt = case
+    say(f"decode scores: H={H} Hkv={Hkv} Q={Q} M={M} D={D} {dt}")
+    g = torch.Generator().manual_seed(71 + M)
+    q = torch.randn(H, Q, D, generator=g).to(dt)
+    k = torch.randn(M, Hkv, D, generator=g).to(dt).transpose(0, 1)
+    invf = base_inv_freq(D, 10000.0)
+    Qs = min(Q, M)
+    plan = native.DecodePlan(q[:, :Qs].to(DEV), k.to(DEV), None, torch.zeros(H), invf, M - Qs, 0.5, 1.0, 0.125, k_max=1)
+    s = plan.scores(torch.full((H, Qs, M), float("nan"), device=DEV)).cpu().double()
+
+    def rot(x, pos):
+        ang = (pos.float() * 0.5)[:, None] * invf
+        c, sn = torch.cos(ang.double()), torch.sin(ang.double())
+        a, b = x[..., :D // 2].double(), x[..., D // 2:].double()
+        return torch.cat((a * c - b * sn, b * c + a * sn), -1)
+
+    qr = rot(q[:, :Qs], torch.arange(M - Qs, M))
+    kr = rot(k, torch.arange(M))
+    for h in range(H):
+        ref = (qr[h] @ kr[h // (H // Hkv)].T) * 0.125
+        bound = 0.125 * qr[h].norm(dim=1)[:, None] * kr[h // (H // Hkv)].norm(dim=1)[None] * 2.0 ** -20
+        for i in range(Qs):
+            m = M - (Qs - 1 - i)
+            assert bool(((s[h, i, :m] - ref[i, :m]).abs() <= bound[i, :m]).all()), f"head {h} query {i}"
