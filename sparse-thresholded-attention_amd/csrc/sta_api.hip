@@ -176,14 +176,10 @@ int run_kernel_a(const sta_shared_args* a, const Layout& L, hipStream_t st) {
   // 16-bit inputs with plain votes score pass 2 with the fp6 correction (sta_fp6.h); fp32 inputs
   // keep the three-product scores throughout
   const bool want6 = a->dtype != STA_DTYPE_F32 && a->select_score == STA_SCORE_FREQ && !a->row_counts;
-  hipError_t e = launch_rope_frag(a->dtype, a->D, a->q, a->q_head_stride, a->q_tok_stride, a->H, a->N,
-                                  L.q_rows_pad, a->q_pos_base, a->pos_scale_a, a->rope_scale_a,
-                                  a->inv_freq_a, qfrag, st, want6);
-  if (e != hipSuccess) return hip_fail(e, "rope pre-kernel (q)");
-  e = launch_rope_frag(a->dtype, a->D, a->k, a->k_head_stride, a->k_tok_stride, a->Hkv, a->N,
-                       L.k_rows_pad, 0, a->pos_scale_a, a->rope_scale_a, a->inv_freq_a, kfrag, st, want6,
-                       (float2*)(ws + L.ktrig_off));
-  if (e != hipSuccess) return hip_fail(e, "rope pre-kernel (k)");
+  const RopeSide rq{a->q, a->q_head_stride, a->q_tok_stride, a->H, a->N, L.q_rows_pad, a->q_pos_base, qfrag, nullptr};
+  const RopeSide rk{a->k, a->k_head_stride, a->k_tok_stride, a->Hkv, a->N, L.k_rows_pad, 0, kfrag, (float2*)(ws + L.ktrig_off)};
+  hipError_t e = launch_rope_frag(a->dtype, a->D, rq, rk, a->pos_scale_a, a->rope_scale_a, a->inv_freq_a, st, want6);
+  if (e != hipSuccess) return hip_fail(e, "rope pre-kernel");
   if ((rc = mark(a, 1, st)) != STA_OK) return rc;
   ScoreArgs sa{};
   sa.qfrag = qfrag;

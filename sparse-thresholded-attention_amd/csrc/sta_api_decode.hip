@@ -160,13 +160,10 @@ int dec_scores(const sta_decode_args* a, const DecLayout& L, DecodeArgs d, float
   char* ws = (char*)a->workspace;
   u32x4* qfrag = (u32x4*)(ws + L.qfrag_off);
   u32x4* kfrag = (u32x4*)(ws + L.kfrag_off);
-  hipError_t e = launch_rope_frag(a->dtype, a->D, a->q, a->q_head_stride, a->q_tok_stride, a->H, a->Q,
-                                  L.q_rows_pad, a->q_pos0, a->pos_scale_a, a->rope_scale_a, a->inv_freq_a,
-                                  qfrag, st);
-  if (e != hipSuccess) return hip_fail(e, "decode scores: rope pre-kernel (q)");
-  e = launch_rope_frag(a->dtype, a->D, a->k, a->k_head_stride, a->k_tok_stride, a->Hkv, a->M, L.k_rows_pad, 0,
-                       a->pos_scale_a, a->rope_scale_a, a->inv_freq_a, kfrag, st);
-  if (e != hipSuccess) return hip_fail(e, "decode scores: rope pre-kernel (k)");
+  const RopeSide rq{a->q, a->q_head_stride, a->q_tok_stride, a->H, a->Q, L.q_rows_pad, a->q_pos0, qfrag, nullptr};
+  const RopeSide rk{a->k, a->k_head_stride, a->k_tok_stride, a->Hkv, a->M, L.k_rows_pad, 0, kfrag, nullptr};
+  hipError_t e = launch_rope_frag(a->dtype, a->D, rq, rk, a->pos_scale_a, a->rope_scale_a, a->inv_freq_a, st);
+  if (e != hipSuccess) return hip_fail(e, "decode scores: rope pre-kernel");
   RowsArgs r{};
   r.qfrag = qfrag;
   r.kfrag = kfrag;

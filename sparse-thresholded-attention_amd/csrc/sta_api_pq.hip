@@ -92,14 +92,10 @@ int pq_run_kernel_a(const sta_pq_args* a, const PqLayout& L, hipStream_t st) {
   u32x4* kfrag = (u32x4*)(ws + L.kfrag_off);
   int rc = mark_event(a->stage_events, 0, st);
   if (rc != STA_OK) return rc;
-  hipError_t e = launch_rope_frag(a->dtype, a->D, a->q, a->q_head_stride, a->q_tok_stride, a->H, a->N,
-                                  L.q_rows_pad, a->q_pos_base, a->pos_scale_a, a->rope_scale_a,
-                                  a->inv_freq_a, qfrag, st);
-  if (e != hipSuccess) return hip_fail(e, "rope pre-kernel (q)");
-  e = launch_rope_frag(a->dtype, a->D, a->k, a->k_head_stride, a->k_tok_stride, a->Hkv, a->N,
-                       L.k_rows_pad, 0, a->pos_scale_a, a->rope_scale_a, a->inv_freq_a, kfrag, st, false,
-                       (float2*)(ws + L.ktrig_off));
-  if (e != hipSuccess) return hip_fail(e, "rope pre-kernel (k)");
+  const RopeSide rq{a->q, a->q_head_stride, a->q_tok_stride, a->H, a->N, L.q_rows_pad, a->q_pos_base, qfrag, nullptr};
+  const RopeSide rk{a->k, a->k_head_stride, a->k_tok_stride, a->Hkv, a->N, L.k_rows_pad, 0, kfrag, (float2*)(ws + L.ktrig_off)};
+  hipError_t e = launch_rope_frag(a->dtype, a->D, rq, rk, a->pos_scale_a, a->rope_scale_a, a->inv_freq_a, st);
+  if (e != hipSuccess) return hip_fail(e, "rope pre-kernel");
   if ((rc = mark_event(a->stage_events, 1, st)) != STA_OK) return rc;
   ScoreArgs sa{};
   sa.qfrag = qfrag;

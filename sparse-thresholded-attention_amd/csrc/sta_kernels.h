@@ -410,12 +410,20 @@ __device__ inline bool fast6_serves(const ScoreArgs& a, int h, int g, int D, int
   return sg <= FAST6_SIGMA_LIMIT;
 }
 
-// want6: also write the fp6 correction operands of the fragment region; trig: also write each
-// row's scaled (cos, sin) pairs, (rows_pad, D/2) float2 (ScoreArgs::ktrig)
-hipError_t launch_rope_frag(int dtype, int D, const void* x, int64_t head_stride, int64_t tok_stride,
-                            int heads, int N, int rows_pad, int pos_base, float pos_scale,
-                            float rope_scale, const float* inv_freq, u32x4* frag, hipStream_t st,
-                            bool want6 = false, float2* trig = nullptr);
+// One side of the selection-geometry RoPE pre-kernel: `heads` heads of N rows (positions pos_base
+// + row) into the fragment region `frag` of rows_pad rows; trig: also write each row's scaled (cos,
+// sin) pairs, (rows_pad, D/2) float2 (ScoreArgs::ktrig)
+struct RopeSide {
+  const void* x;
+  int64_t head_stride, tok_stride;
+  int heads, N, rows_pad, pos_base;
+  u32x4* frag;
+  float2* trig;
+};
+// queries and keys in one launch, then their norm maxima in another; want6: also write the fp6
+// correction operands of the fragment regions
+hipError_t launch_rope_frag(int dtype, int D, const RopeSide& q, const RopeSide& k, float pos_scale,
+                            float rope_scale, const float* inv_freq, hipStream_t st, bool want6 = false);
 // the fp6 pass-2 kernel (plain votes); the launcher of the score passes calls it
 hipError_t launch_score6(int D, int tile, const ScoreArgs& a, hipStream_t st);
 hipError_t launch_score(int D, int tile, const ScoreArgs& a, hipStream_t st);

@@ -155,30 +155,48 @@ __device__ __forceinline__ void write_fp6(const float* o1, const float* o2, cons
   if (c == 0) dnorms6[(int64_t)head * rows_pad + row] = make_float2(sqrtf(dh), sqrtf(dr));
 }
 
+// what the kernel reads and writes of one side (RopeSide): blockIdx.y < ny of the first side, then
+// the second's
+struct RopeJob {
+  const void* x;
+  int64_t head_stride, tok_stride;
+  int heads, N, rows_pad, pos_base, ny;
+  u32x4* frag;
+  float2* norms;
+  uint32_t* rowkeys;
+  uint64_t* planes6;
+  uint32_t* scales6;
+  float2* dnorms6;
+  float2* trig;
+};
+
 template <int DT, int D, bool W6>
-__global__ __launch_bounds__(256) void rope_frag_kernel(const void* __restrict__ x, int64_t head_stride,
-                                                        int64_t tok_stride, int heads, int N, int rows_pad,
-                                                        int pos_base, float pos_scale, float rope_scale,
-                                                        const float* __restrict__ inv_freq,
-                                                        u32x4* __restrict__ frag, float2* __restrict__ norms,
-                                                        uint64_t* __restrict__ planes6, uint32_t* __restrict__ scales6,
-                                                        float2* __restrict__ dnorms6, float2* __restrict__ trig,
-                                                        uint32_t* __restrict__ rowkeys) {
+__global__ __launch_bounds__(256) void rope_frag_kernel(RopeJob jq, RopeJob jk, float pos_scale, float rope_scale,
+                                                        const float* __restrict__ inv_freq) {
 #pragma clang fp contract(off)
   constexpr int C2 = D / 16;                 // threads per row
+  const bool second = (int)blockIdx.y >= jq.ny;
+  const RopeJob& j = second ? jk : jq;
+  const void* __restrict__ x = j.x;
+  const int64_t head_stride = j.head_stride, tok_stride = j.tok_stride;
+  const int N = j.N, rows_pad = j.rows_pad;
+  u32x4* __restrict__ frag = j.frag;
+  float2* __restrict__ norms = j.norms;
+  float2* __restrict__ trig = j.trig;
   const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
   // the fp6 operands' row exchange (LDS, per wave: rows never span waves)
   __shared__ float lds6[4][W6 ? Fp6Rows<D>::ROWS * Fp6Rows<D>::RS : 1];
   if (gid >= (int64_t)rows_pad * C2) return;
   const int c = (int)(gid % C2);
   const int row = (int)(gid / C2);
-  const int h0 = blockIdx.y * ROPE_HG;
-  const int h1 = h0 + ROPE_HG < heads ? h0 + ROPE_HG : heads;
+  const int by = (int)blockIdx.y - (second ? jq.ny : 0);
+  const int h0 = by * ROPE_HG;
+  const int h1 = min(h0 + ROPE_HG, j.heads);
   const int i0 = c * 8;
   const bool live = row < N;
   float cs[8], sn[8];
   if (live) {
-    const float pf = (float)(pos_base + row) * pos_scale;
+    const float pf = (float)(j.pos_base + row) * pos_scale;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float ang = pf * inv_freq[i0 + e];
@@ -188,7 +206,7 @@ __global__ __launch_bounds__(256) void rope_frag_kernel(const void* __restrict__
     }
     // the row's (cos, sin) table, written once (first head group): the screened pass 1 rebuilds
     // a candidate key's fragments from its raw row and this table, 2 + 4 cache lines per key
-    if (trig && blockIdx.y == 0) {
+    if (trig && by == 0) {
       float4* t = (float4*)(trig + (int64_t)row * (D / 2) + i0);
 #pragma unroll
       for (int e = 0; e < 4; ++e) t[e] = make_float4(cs[2 * e], sn[2 * e], cs[2 * e + 1], sn[2 * e + 1]);
@@ -249,22 +267,30 @@ __global__ __launch_bounds__(256) void rope_frag_kernel(const void* __restrict__
     }
     if (c == 0) {
       norms[(int64_t)head * rows_pad + row] = make_float2(sqrtf(sh), sqrtf(sl));
-      rowkeys[(int64_t)head * rows_pad + row] = 0u;   // the key-split pass 1 merges its row maxima here
+      j.rowkeys[(int64_t)head * rows_pad + row] = 0u;   // the key-split pass 1 merges its row maxima here
     }
-    if constexpr (W6) write_fp6<D>(o1, o2, hi1, hi2, c, row, head, rows_pad, lds6[threadIdx.x >> 6], planes6, scales6, dnorms6);
+    if constexpr (W6) write_fp6<D>(o1, o2, hi1, hi2, c, row, head, rows_pad, lds6[threadIdx.x >> 6], j.planes6, j.scales6,
+                                  j.dnorms6);
   }
 }
 
-// per head: the maxima of (||hi||, ||lo||) over its rows_pad rows (rows_pad even); 1024 threads
-// read two rows per 16-byte load, several loads in flight per thread.  blockIdx.y picks one of two
-// (norms, out) pairs, so the fp6 rounding norms take the same launch.
-__global__ __launch_bounds__(1024) void norm_max_kernel(const float2* __restrict__ norms0, float2* __restrict__ out0,
-                                                        const float2* __restrict__ norms1, float2* __restrict__ out1,
-                                                        int rows_pad) {
+// per head of both sides: the maxima of (||hi||, ||lo||) over its rows_pad rows (rows_pad even); 1024
+// threads read two rows per 16-byte load, several loads in flight per thread.  blockIdx.x: the first
+// side's heads, then the second's; blockIdx.y 1: the fp6 rounding norms instead.
+struct NormJob {
+  const float2* norms[2];   // (heads, rows_pad): the rows' norms, the fp6 rounding norms
+  float2* out[2];           // (heads,)
+  int heads, rows_pad;
+};
+
+__global__ __launch_bounds__(1024) void norm_max_kernel(NormJob jq, NormJob jk) {
   __shared__ float red[2][16];
-  const int head = blockIdx.x, tid = threadIdx.x;
-  const float2* norms = blockIdx.y == 0 ? norms0 : norms1;
-  float2* out = blockIdx.y == 0 ? out0 : out1;
+  const bool second = (int)blockIdx.x >= jq.heads;
+  const NormJob& j = second ? jk : jq;
+  const int head = (int)blockIdx.x - (second ? jq.heads : 0), tid = threadIdx.x;
+  const int rows_pad = j.rows_pad;
+  const float2* norms = j.norms[blockIdx.y];
+  float2* out = j.out[blockIdx.y];
   const float4* p = (const float4*)(norms + (int64_t)head * rows_pad);
   const int n4 = rows_pad / 2;
   float mh = 0.0f, ml = 0.0f;
@@ -1388,37 +1414,37 @@ void score_kernel(ScoreArgs a) {
 // host launchers
 // ------------------------------------------------------------------------------------------
 template <int DT, int D>
-static hipError_t launch_rope_frag_t(const void* x, int64_t hs, int64_t ts, int heads, int N, int rows_pad,
-                                     int pos_base, float pos_scale, float rope_scale, const float* inv_freq,
-                                     u32x4* frag, hipStream_t st, bool want6, float2* trig) {
-  const int64_t total = (int64_t)rows_pad * (D / 16);
-  const int64_t blocks = (total + 255) / 256;
-  float2* norms = frag_norms(frag, heads, rows_pad, D);
-  uint32_t* rowkeys = (uint32_t*)frag_rowmax(frag, heads, rows_pad, D);
-  uint64_t* planes6 = want6 ? frag6_planes(frag, heads, rows_pad, D) : nullptr;
-  uint32_t* scales6 = frag6_scales(frag, heads, rows_pad, D);
-  float2* dn6 = frag6_dnorms(frag, heads, rows_pad, D);
-  const dim3 grid((unsigned)blocks, (unsigned)((heads + ROPE_HG - 1) / ROPE_HG));
+static hipError_t launch_rope_frag_t(const RopeSide& q, const RopeSide& k, float pos_scale, float rope_scale,
+                                     const float* inv_freq, hipStream_t st, bool want6) {
+  auto job = [&](const RopeSide& s) {
+    return RopeJob{s.x, s.head_stride, s.tok_stride, s.heads, s.N, s.rows_pad, s.pos_base,
+                   (s.heads + ROPE_HG - 1) / ROPE_HG, s.frag, frag_norms(s.frag, s.heads, s.rows_pad, D),
+                   (uint32_t*)frag_rowmax(s.frag, s.heads, s.rows_pad, D),
+                   want6 ? frag6_planes(s.frag, s.heads, s.rows_pad, D) : nullptr,
+                   frag6_scales(s.frag, s.heads, s.rows_pad, D), frag6_dnorms(s.frag, s.heads, s.rows_pad, D), s.trig};
+  };
+  auto norm = [&](const RopeSide& s) {
+    return NormJob{{frag_norms(s.frag, s.heads, s.rows_pad, D), frag6_dnorms(s.frag, s.heads, s.rows_pad, D)},
+                   {frag_norm_max(s.frag, s.heads, s.rows_pad, D), frag6_dnorm_max(s.frag, s.heads, s.rows_pad, D)},
+                   s.heads, s.rows_pad};
+  };
+  const RopeJob jq = job(q), jk = job(k);
+  const int64_t rows = q.rows_pad > k.rows_pad ? q.rows_pad : k.rows_pad;
+  const dim3 grid((unsigned)((rows * (D / 16) + 255) / 256), (unsigned)(jq.ny + jk.ny));
   if (want6)
-    hipLaunchKernelGGL((rope_frag_kernel<DT, D, true>), grid, dim3(256), 0, st, x, hs, ts, heads, N,
-                       rows_pad, pos_base, pos_scale, rope_scale, inv_freq, frag, norms, planes6, scales6, dn6, trig, rowkeys);
+    hipLaunchKernelGGL((rope_frag_kernel<DT, D, true>), grid, dim3(256), 0, st, jq, jk, pos_scale, rope_scale, inv_freq);
   else
-    hipLaunchKernelGGL((rope_frag_kernel<DT, D, false>), grid, dim3(256), 0, st, x, hs, ts, heads, N,
-                       rows_pad, pos_base, pos_scale, rope_scale, inv_freq, frag, norms, planes6, scales6, dn6, trig, rowkeys);
-  hipError_t e = hipGetLastError();
+    hipLaunchKernelGGL((rope_frag_kernel<DT, D, false>), grid, dim3(256), 0, st, jq, jk, pos_scale, rope_scale, inv_freq);
+  const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  // the row norms' maxima, and with the fp6 planes their rounding norms' in the same launch
-  hipLaunchKernelGGL(norm_max_kernel, dim3(heads, want6 ? 2 : 1), dim3(1024), 0, st, (const float2*)norms,
-                     frag_norm_max(frag, heads, rows_pad, D), (const float2*)dn6,
-                     frag6_dnorm_max(frag, heads, rows_pad, D), rows_pad);
+  hipLaunchKernelGGL(norm_max_kernel, dim3(q.heads + k.heads, want6 ? 2 : 1), dim3(1024), 0, st, norm(q), norm(k));
   return hipGetLastError();
 }
 
-hipError_t launch_rope_frag(int dtype, int D, const void* x, int64_t hs, int64_t ts, int heads, int N,
-                            int rows_pad, int pos_base, float pos_scale, float rope_scale,
-                            const float* inv_freq, u32x4* frag, hipStream_t st, bool want6, float2* trig) {
+hipError_t launch_rope_frag(int dtype, int D, const RopeSide& q, const RopeSide& k, float pos_scale,
+                            float rope_scale, const float* inv_freq, hipStream_t st, bool want6) {
 #define STA_RF(DT_, D_) \
-  if (dtype == DT_ && D == D_) return launch_rope_frag_t<DT_, D_>(x, hs, ts, heads, N, rows_pad, pos_base, pos_scale, rope_scale, inv_freq, frag, st, want6, trig);
+  if (dtype == DT_ && D == D_) return launch_rope_frag_t<DT_, D_>(q, k, pos_scale, rope_scale, inv_freq, st, want6);
   STA_RF(DT_F32, 64) STA_RF(DT_F32, 128) STA_RF(DT_BF16, 64) STA_RF(DT_BF16, 128)
   STA_RF(DT_F16, 64) STA_RF(DT_F16, 128)
 #undef STA_RF
