@@ -75,7 +75,8 @@ def decode_attention(q, k, v, tau, inv_freq, q_pos0, pos_scale=1.0, rope_scale=1
         sm_scale = 1.0 / math.sqrt(qh.shape[-1])
     r = native.decode_attention(qh, k, v, _tau_of(tau, qh.shape[0]), inv_freq, q_pos0, pos_scale, rope_scale,
                                 sm_scale, n_global, n_local, k_max, pct_decode, causal, inv_freq_c=inv_freq_c,
-                                pos_scale_c=pos_scale_c, rope_scale_c=rope_scale_c, rule=rule, block_n=block_n)
+                                pos_scale_c=pos_scale_c, rope_scale_c=rope_scale_c, rule=rule, block_n=block_n,
+                                sets=stats is not None)
     if stats is not None and rule == "pq":
         stats["usize"], stats["overflow"] = r["usize"], r["overflow"]
     if stats is not None and rule == "stream":

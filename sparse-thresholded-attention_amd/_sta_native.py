@@ -280,7 +280,9 @@ def _heads_view(x):
 
 
 def _stream(dev):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    # the raw handle: torch.cuda.current_stream(dev).cuda_stream without the Stream object (2.1 us a call)
+    index = torch.cuda.current_device() if dev.index is None else dev.index
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(index))
 
 
 def start_pct_of(pct):
@@ -1076,14 +1078,17 @@ class DecodePlan:
 
     def __init__(self, q, k, v, tau, inv_freq, q_pos0, pos_scale=1.0, rope_scale=1.0, sm_scale=None,
                  n_global=32, n_local=32, k_max=1024, pct_decode=100.0, causal=False, want_scores=False,
-                 inv_freq_c=None, pos_scale_c=None, rope_scale_c=None, rule="shared", block_n=32):
+                 inv_freq_c=None, pos_scale_c=None, rope_scale_c=None, rule="shared", block_n=32, sets=True):
         """inv_freq / pos_scale / rope_scale: the selection geometry; the *_c triple (default: the
         same) repositions (pos_scale_c) and attends (inv_freq_c, rope_scale_c).  rule "shared" is
         _decode_build_sets (exact_2.py:527-604), "pq" _decode_build_sets_pq (perquery.py:651-720:
         dense ranks, exact cap budget; pass rope_scale_c=1 and the base inv_freq_c); "pq" also
         fills usize and overflow (H, Q).  "stream" is _decode_build_sets_pqs (pqstream_kernel.py:
         695-797: every passer and forced key, no cap, streamed positions over blocks of block_n
-        keys walked back from the query; k_max is the slot buffer, M rounded up to 1024)."""
+        keys walked back from the query; k_max is the slot buffer, M rounded up to 1024).
+        sets=False: self.out holds `out` alone and the set arrays lie behind the workspace, in its
+        allocation.  A call that builds a plan on a small cache is bound by the host (8 kv heads x
+        2000 keys, one query a head: 40 -> 27 us a call), and an allocation takes 1.8 us."""
         if not q.is_cuda:
             raise RuntimeError("sparse-thresholded attention runs on a HIP device only; got a CPU tensor")
         if q.dtype not in DTYPES:
@@ -1123,27 +1128,36 @@ class DecodePlan:
         a.rule = RULES[rule]
         a.block_n = int(block_n)
         self._keep = (qh, kh, vh, tau, ifr, ifc)
-        self.out = {
-            "out": torch.empty((H, Q, D), dtype=qh.dtype, device=dev),
-            "idx": torch.empty((H, Q, k_max), dtype=torch.int32, device=dev),
-            "newpos_k": torch.empty((H, Q, k_max), dtype=torch.float32, device=dev),
-            "newpos_q": torch.empty((H, Q), dtype=torch.float32, device=dev),
-            "set_size": torch.empty((H, Q), dtype=torch.int32, device=dev),
-        }
+        self.out = {"out": torch.empty((H, Q, D), dtype=qh.dtype, device=dev)}
+        a.out = self.out["out"].data_ptr()
+        if sets:
+            self.out["idx"] = torch.empty((H, Q, k_max), dtype=torch.int32, device=dev)
+            self.out["newpos_k"] = torch.empty((H, Q, k_max), dtype=torch.float32, device=dev)
+            self.out["newpos_q"] = torch.empty((H, Q), dtype=torch.float32, device=dev)
+            self.out["set_size"] = torch.empty((H, Q), dtype=torch.int32, device=dev)
+            if rule == "pq":
+                self.out["usize"] = torch.empty((H, Q), dtype=torch.int32, device=dev)
+                self.out["overflow"] = torch.empty((H, Q), dtype=torch.bool, device=dev)
+            for name in ("idx", "newpos_k", "newpos_q", "set_size"):
+                setattr(a, name, _ptr(self.out[name]))
+            a.usize, a.overflow = _ptr(self.out.get("usize")), _ptr(self.out.get("overflow"))
         if want_scores:
             self.out["scores"] = torch.empty((H, Q, M), dtype=torch.float32, device=dev)
-        if rule == "pq":
-            self.out["usize"] = torch.empty((H, Q), dtype=torch.int32, device=dev)
-            self.out["overflow"] = torch.empty((H, Q), dtype=torch.bool, device=dev)
-        for name in ("out", "idx", "newpos_k", "newpos_q", "set_size"):
-            setattr(a, name, _ptr(self.out[name]))
-        a.scores = _ptr(self.out.get("scores"))
-        a.usize, a.overflow = _ptr(self.out.get("usize")), _ptr(self.out.get("overflow"))
+            a.scores = _ptr(self.out["scores"])
         n = lib().sta_decode_workspace_size(ctypes.byref(a))
         if n == 0:
             _check(-1, "sta_decode_workspace_size")
-        self.workspace = torch.empty(n, dtype=torch.uint8, device=dev)
-        a.workspace, a.workspace_bytes = _ptr(self.workspace), n
+        if sets:
+            self.workspace = torch.empty(n, dtype=torch.uint8, device=dev)
+            a.workspace = self.workspace.data_ptr()
+        else:
+            base = -(-n // 256) * 256
+            rows, slots = -(-4 * H * Q // 256) * 256, -(-4 * H * Q * k_max // 256) * 256
+            self.workspace = torch.empty(base + 2 * slots + 2 * rows, dtype=torch.uint8, device=dev)
+            a.workspace = p = self.workspace.data_ptr()
+            a.idx, a.newpos_k = p + base, p + base + slots
+            a.newpos_q, a.set_size = p + base + 2 * slots, p + base + 2 * slots + rows
+        a.workspace_bytes = n
         self._events = None
 
     def run(self, events=None):
@@ -1200,14 +1214,14 @@ class DecodePlan:
 
 def decode_attention(q, k, v, tau, inv_freq, q_pos0, pos_scale=1.0, rope_scale=1.0, sm_scale=None,
                      n_global=32, n_local=32, k_max=1024, pct_decode=100.0, causal=False, want_scores=False,
-                     inv_freq_c=None, pos_scale_c=None, rope_scale_c=None, rule="shared", block_n=32):
+                     inv_freq_c=None, pos_scale_c=None, rope_scale_c=None, rule="shared", block_n=32, sets=True):
     """Scores, selection and attend of Q queries (H, Q, D) over the cache k, v (Hkv, M, D).
-    Returns a dict of device tensors: out (H, Q, D), idx (H, Q, k_max) int32 (sentinel m_i),
-    newpos_k, newpos_q, set_size, with want_scores scores (H, Q, M), and under rule "pq" usize
-    and overflow (H, Q)."""
+    Returns a dict of device tensors: out (H, Q, D), with want_scores scores (H, Q, M), and unless
+    sets=False idx (H, Q, k_max) int32 (sentinel m_i), newpos_k, newpos_q, set_size, and under rule
+    "pq" usize and overflow (H, Q)."""
     return DecodePlan(q, k, v, tau, inv_freq, q_pos0, pos_scale, rope_scale, sm_scale, n_global, n_local,
                       k_max, pct_decode, causal, want_scores, inv_freq_c, pos_scale_c, rope_scale_c,
-                      rule, block_n).run()
+                      rule, block_n, sets).run()
 
 
 class PerQueryPrefillPlan:

@@ -361,3 +361,28 @@ def test_decode_scores_over_heads_per_workgroup(case):
         for i in range(Qs):
             m = M - (Qs - 1 - i)
             assert bool(((s[h, i, :m] - ref[i, :m]).abs() <= bound[i, :m]).all()), f"head {h} query {i}"
+
+
+@pytest.mark.parametrize("rule", ["shared", "pq", "stream"])
+@pytest.mark.parametrize("H,Hkv,Q,M,km", [(3, 1, 1, 40, 65), (8, 2, 5, 700, 129)])
+def test_decode_without_set_arrays(rule, H, Hkv, Q, M, km):
+    """The call that returns the output alone keeps its sets behind the workspace: same bits."""
+    import _sta_native as native
+    from _decode import decode_attention
+    say(f"decode, output alone: {rule} H={H} Hkv={Hkv} Q={Q} M={M}")
+    km = 1024 if rule == "stream" else km
+    g = torch.Generator().manual_seed(5)
+    q = torch.randn(1, H, Q, 64, generator=g).to(DEV)
+    k, v = (torch.randn(1, Hkv, M, 64, generator=g).to(DEV) for _ in range(2))
+    invf = (10000.0 ** (-torch.arange(0, 64, 2) / 64.0)).to(DEV)
+    tau = torch.full((H,), 2.0, device=DEV)
+    args = (tau, invf, M - Q, 1.0, 1.0, None, 8, 8, km)
+    r = native.decode_attention(q, k, v, *args, rule=rule)
+    stats = {}
+    with_stats = decode_attention(q, k, v, *args, rule=rule, stats=stats)
+    plan = native.DecodePlan(q, k, v, *args, rule=rule, sets=False)
+    assert set(plan.run()) == {"out"}
+    for out in (plan.run()["out"], decode_attention(q, k, v, *args, rule=rule), with_stats):
+        assert torch.equal(out, r["out"])
+    for name in stats:
+        assert torch.equal(stats[name], r[name])
