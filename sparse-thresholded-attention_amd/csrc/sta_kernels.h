@@ -401,9 +401,8 @@ __device__ inline bool fast6_serves(const ScoreArgs& a, int h, int g, int D, int
   const int rows_total = a.q_rows_pad;
   constexpr int SG = 256;
   const int ng_s = (rows_total + SG - 1) / SG;
-  if (!a.keys1)
-    for (int gs = g * wg_rows / SG; gs < min((g + 1) * wg_rows / SG, ng_s); ++gs)
-      if (a.sflags[h * ng_s + gs] != 0) return false;
+  for (int gs = g * wg_rows / SG; gs < min((g + 1) * wg_rows / SG, ng_s); ++gs)
+    if (a.sflags[h * ng_s + gs] != 0) return false;
   const int kvh = h / (a.H / a.Hkv);
   const float2 qn = a.qnorm_max[h], kn = a.knorm_max[kvh], qd = a.q6dmax[h], kd = a.k6dmax[kvh];
   const float sg = fast6_sigma(qn.x, qn.y, qd.x, qd.y, kn.x, kn.y, kd.x, kd.y, a.sm_scale, D);

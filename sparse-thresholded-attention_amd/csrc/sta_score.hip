@@ -1562,7 +1562,10 @@ static hipError_t launch_score_t(const ScoreArgs& a0, hipStream_t st) {
     // the four products of every score cost what the screen's candidate phase does (32 heads:
     // rows 2000 275 us a call against 294, 3000 399 against 391, 4500 760 against 646; 8 heads x
     // 2048, D 64, fp32: 120 against 202).
-    a.keys1 = !screen_pass1_forced() && chunk_steps(a.H, a.q_pos_base, rows, 32 * RB * WS) <= 8192;
+    // Calls whose pass 2 may run in fp6 keep the screen: its flags hold the row groups with tied or
+    // concentrated scores on the three-product pass 2 (bf16, plain votes, 32 heads x 1000: 157 us a
+    // call where the split pass 1 took 127, 8 x 5632: 354 against 394).
+    a.keys1 = !a.fast6 && !screen_pass1_forced() && chunk_steps(a.H, a.q_pos_base, rows, 32 * RB * WS) <= 8192;
     if (a.keys1) set_split(split_chunks(a.H, a.q_pos_base, rows, 32 * RB * WS, D, WS));
     // the same for every pass-2 epilogue: one instance per (D, T)
     if (a.keys1)

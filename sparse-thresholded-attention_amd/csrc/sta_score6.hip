@@ -115,7 +115,7 @@ __global__ __launch_bounds__(512, 1) void score6_kernel(ScoreArgs a) {
     const int row = wrow0 + lane;
     const bool ok = active && row < a.N;       // padded rows never vote (exact_2.py:121)
     const int64_t ri = (int64_t)h * a.q_rows_pad + (row < rows_total ? row : 0);
-    const float v = row_max_of(a, ri);
+    const float v = a.srmax[ri];
     const float m = v * a.sm_scale;            // fl(max * c) == max of fl(s * c) for c > 0
     float x = ok ? min_arg_for(m - tau, a.sm_scale) : INFINITY;
     if (ok && tau >= 0.0f) {

@@ -1,7 +1,8 @@
 """GPU: score passes whose keys are split over workgroups.
 
-Short calls take pass 1 as a sweep of every score in the screen's four products, each row group's
-keys split over workgroups and the row maxima merged; grids of few row groups split pass 2's keys.
+Short calls, but those whose pass 2 may run in fp6 (16-bit inputs, plain votes), take pass 1 as a
+sweep of every score in the screen's four products, each row group's keys split over workgroups and
+the row maxima merged; grids of few row groups split pass 2's keys.
 The maximum is over the same fp32 values and a key's votes need no other key, so both agree with
 the unsplit kernels bit for bit: with the screened pass 1 (STA_SCREEN_PASS1=1), and with the
 row-count instances of pass 2, which stay whole.
@@ -108,3 +109,28 @@ def test_rows_and_keys_that_are_not_finite(monkeypatch):
     assert np.array_equal(fine, np.isfinite(ma))
     assert np.abs(ma[fine] - mb[fine]).max() < 1e-4
     assert (va != vb).mean() < 1e-4
+
+
+@pytest.mark.parametrize("dt,tile", [(torch.bfloat16, 64), (torch.float16, 32)])
+def test_concentrated_scores_keep_three_products(dt, tile, monkeypatch):
+    """Keys that differ by 2% of their size: the screen cannot single out a row's maximum anywhere, so
+    plain votes of 16-bit inputs take three products in both passes, as under STA_EXACT_PASS1=1, bit
+    for bit (the fp6 correction moves hundreds of these votes)."""
+    import _sta_native as native
+    from synthetic import base_inv_freq
+    H, N, D = 2, 1500, 128
+    say(f"concentrated scores, plain votes: {dt} tile={tile}")
+    g = torch.Generator().manual_seed(47)
+    q = torch.randn(1, H, N, D, generator=g).to(dt).to(DEV)
+    k = (torch.randn(1, H, 1, D, generator=g) + 0.02 * torch.randn(1, H, N, D, generator=g)).to(dt).to(DEV)
+    invf = base_inv_freq(D, 10000.0).to(DEV)
+    tau = torch.full((H,), 0.03)
+    got = []
+    for exact in ("0", "1"):
+        monkeypatch.setenv("STA_EXACT_PASS1", exact)
+        votes, _, rm = native.select_vote(q, k, tau, invf, 0.0, 1.1, 1.0 / math.sqrt(D), tile, want_row_counts=False)
+        torch.cuda.synchronize()
+        got.append((votes.cpu().numpy(), rm.cpu().numpy()))
+    (va, ma), (vb, mb) = got
+    assert va.sum() > 10000
+    assert np.array_equal(ma, mb) and np.array_equal(va, vb), f"{int((va != vb).sum())} vote entries differ"
