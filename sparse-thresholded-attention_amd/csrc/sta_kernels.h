@@ -77,6 +77,8 @@ struct ScoreArgs {
   int* sflags;            // (H, ngroups) the screen's fallback flags
   int keys1;              // set by the launcher: pass 1 ran as the key-split sweep, and srmax holds
                           // order keys (row_key) instead of floats; sflags is not written
+  int swept;              // set by the launcher: behind the screen, the key-split sweep left order keys
+                          // in srmax for the row groups with sflags (without the screen: for all)
   int pieces, pchunks;    // set by the launcher, per launch: a row group's 64-key chunks are split
                           // over `pieces` workgroups of at most `pchunks` chunks each
   float* xthr;            // thresholds-only instance: (H, q_rows_pad) each row's x0 (+inf: no row)
@@ -369,11 +371,6 @@ __device__ __forceinline__ uint32_t row_key(float v) {
 __device__ __forceinline__ float row_key_value(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
 }
-// the raw maximum of fragment row i (of H * q_rows_pad) as pass 1 left it
-__device__ __forceinline__ float row_max_of(const ScoreArgs& a, int64_t i) {
-  return a.keys1 ? row_key_value(((const uint32_t*)a.srmax)[i]) : a.srmax[i];
-}
-
 // Workgroup `bid` of H heads x ngroups row groups x pieces key pieces.  XCD-aware: workgroup i runs
 // on XCD i % 8, so with H a multiple of 8 a head stays on one XCD; the heaviest groups come first.
 __device__ __forceinline__ void score_workgroup(int bid, int H, int ngroups, int pieces, int& h, int& g, int& piece) {

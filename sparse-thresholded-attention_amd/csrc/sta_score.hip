@@ -425,6 +425,10 @@ void score_kernel(ScoreArgs a) {
   const int nall = (hi_max + CK - 1) / CK;
   const int nchunks = MODE == 1 ? nall : min(nall, c0 + a.pchunks);
   if (c0 >= nchunks) return;
+  // MODE 2 behind the screen: the row groups that it gave up
+  if constexpr (MODE == 2) {
+    if (!a.keys1 && a.screened && a.sflags[h * ngroups + g] == 0) return;
+  }
   // chunks entirely below N whose keys are causal for every query of the workgroup
   const int nfull_all = min(min(nall, (a.q_pos_base + g * WG_ROWS + 1) / CK), a.N / CK);
   const int nfull = min(nfull_all, nchunks);
@@ -564,11 +568,12 @@ void score_kernel(ScoreArgs a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) { ref[rb][i] = 0.0f; rc[rb][i] = 0; }
 
-  // 32 keys x this wave's rows, one k step: hi.hi + hi.lo + lo.hi, small terms first; MODE 2: the
+  // The sweeps: pass 0 takes row maxima and pass 1 votes, both over three products a score; pass 2
+  // takes row maxima over the screen's four.
+  // 32 keys x this wave's rows, one k step: hi.hi + hi.lo + lo.hi, small terms first; pass 2: the
   // screen's four products in its order
-  constexpr int NPROD = MODE == 2 ? 4 : 3;
-  auto mfma3 = [&](u32x4 bh, u32x4 bl, int s, floatx16* acc) {
-    if constexpr (MODE == 2) {
+  auto mfma3 = [&](auto passc, u32x4 bh, u32x4 bl, int s, floatx16* acc) {
+    if constexpr (decltype(passc)::value == 2) {
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) acc[rb] = mfma32(qhi[rb][s], bh, acc[rb]);
 #pragma unroll
@@ -592,8 +597,9 @@ void score_kernel(ScoreArgs a) {
   // interleaved between the MFMAs.  One wave per SIMD has no other wave to hide LDS latency.  The
   // reads for step s + 2 follow step s + 1's first MFMA, so the LDS wait in front of that MFMA
   // covers only reads issued a whole step earlier.
-  auto block_schedule = [&](auto valuc) {
+  auto block_schedule = [&](auto passc, auto valuc) {
     constexpr int valu_per_mfma = decltype(valuc)::value;
+    constexpr int NPROD = decltype(passc)::value == 2 ? 4 : 3;
     __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);        // reads of steps 0 and 1
 #pragma unroll
     for (int s = 0; s < S; ++s) {
@@ -606,22 +612,22 @@ void score_kernel(ScoreArgs a) {
     }
   };
   // all k steps of block sb, with the next step's K fragments read ahead
-  auto mfma_block = [&](const u32x4* buf, int sb, floatx16* acc) {
+  auto mfma_block = [&](auto passc, const u32x4* buf, int sb, floatx16* acc) {
     u32x4 bh = ldb(buf, sb, 0, 0), bl = ldb(buf, sb, 0, 1);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       u32x4 nh = bh, nl = bl;
       if (s + 1 < S) { nh = ldb(buf, sb, s + 1, 0); nl = ldb(buf, sb, s + 1, 1); }
-      mfma3(bh, bl, s, acc);
+      mfma3(passc, bh, bl, s, acc);
       bh = nh;
       bl = nl;
     }
-    block_schedule(std::integral_constant<int, 0>{});
+    block_schedule(passc, std::integral_constant<int, 0>{});
   };
   // epilogue of one (unmasked) score
   auto epi = [&](auto passc, float v, int rb, int i, int* cnt, uint32_t* bm, float* w) {
     constexpr int pass = decltype(passc)::value;
-    if constexpr (pass == 0) {
+    if constexpr (pass != 1) {
       mx[rb][i] = __builtin_amdgcn_fmed3f(v, mx[rb][i], pinf);   // max; scores are finite
     } else if constexpr (PLAIN) {
       // rows dropped: the sign of v - x0 (exact: two distinct floats never subtract to zero,
@@ -649,7 +655,7 @@ void score_kernel(ScoreArgs a) {
     for (int s = 0; s < S; ++s) {
       u32x4 nh = bh, nl = bl;
       if (s + 1 < S) { nh = ldb(buf, sb, s + 1, 0); nl = ldb(buf, sb, s + 1, 1); }
-      mfma3(bh, bl, s, accN);
+      mfma3(passc, bh, bl, s, accN);
       bh = nh;
       bl = nl;
       if constexpr (HAS_PREV) {
@@ -667,7 +673,7 @@ void score_kernel(ScoreArgs a) {
       }
       store_key(keyO + (lane & 31), false, cnt, bm, w);
     }
-    block_schedule(std::integral_constant<int, HAS_PREV ? 2 : 0>{});
+    block_schedule(passc, std::integral_constant<int, HAS_PREV ? 2 : 0>{});
   };
   // Pass 2 of the 8-wave workgroups on fully causal chunks: one row block's MFMAs at a time, the
   // other row block's vote epilogue interleaved between them (two accumulators; the epilogue of
@@ -1218,7 +1224,7 @@ void score_kernel(ScoreArgs a) {
     constexpr int pass = decltype(passc)::value;
     constexpr std::integral_constant<bool, true> kPrev{};
     constexpr std::integral_constant<bool, false> kNoPrev{};
-    if constexpr (pass == 0) {
+    if constexpr (pass != 1) {
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
@@ -1300,7 +1306,7 @@ void score_kernel(ScoreArgs a) {
             floatx16 acc[RB];
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) acc[rb] = floatx16{};
-            mfma_block(buf, sb, acc);
+            mfma_block(passc, buf, sb, acc);
             const int key = key0 + (lane & 31);
             const int dk = key - qpos0 - (lane >> 5) * 4;   // causal: dk <= the slot's row constant
             const bool diag = key0 + 31 > qpos0;
@@ -1313,7 +1319,7 @@ void score_kernel(ScoreArgs a) {
               for (int i = 0; i < 16; ++i) {
                 const bool causal = !diag || dk <= rb * 32 + (i >> 2) * 8 + (i & 3);   // exact_2.py:101, 119
                 const float v = acc[rb][i];
-                if constexpr (pass == 0) {
+                if constexpr (pass != 1) {
                   if (causal && v > mx[rb][i]) mx[rb][i] = v;
                 } else if constexpr (PLAIN) {
                   cnt[rb] += causal ? (int)(__float_as_uint(v - mx[rb][i]) >> 31) : 1;
@@ -1353,23 +1359,33 @@ void score_kernel(ScoreArgs a) {
     }
     return;
   } else if constexpr (MODE == 2) {
-    run_pass(std::integral_constant<int, 0>{}, c0, nchunks);
+    if (a.keys1) run_pass(std::integral_constant<int, 2>{}, c0, nchunks);
+    else run_pass(std::integral_constant<int, 0>{}, c0, nchunks);
     const float v = swept_max();
     if (active && wrow0 + lane < rows_total)
       atomicMax((uint32_t*)a.srmax + (int64_t)h * a.q_rows_pad + wrow0 + lane, row_key(v));
   } else {
-    // pass 1: the screen's row maxima, or the three-product sweep where it fell back or is off
+    // pass 1: the row maxima that the screen or the key-split sweep left, or the three-product sweep
+    // here where the screen fell back or is off
     // the screen's workgroups covering this one's rows (4 waves of 32 RB rows each)
-    bool screen_ok = a.screened;
-    if (!a.keys1) {
+    bool ready = a.keys1 || a.swept, own = a.screened;
+    if (!a.keys1 && a.screened) {
       constexpr int SG = score_waves<false, 0, 1>() * 32 * RB;
       const int ng_s = (rows_total + SG - 1) / SG;
+      bool all = true;
       for (int gs = g * WG_ROWS / SG; gs < min((g + 1) * WG_ROWS / SG, ng_s); ++gs)
-        screen_ok = screen_ok && a.sflags[h * ng_s + gs] == 0;
+        all = all && a.sflags[h * ng_s + gs] == 0;
+      ready = ready || all;
+      own = active && a.sflags[h * ng_s + wrow0 / SG] == 0;   // this wave's rows kept the screen's maxima
     }
-    if (screen_ok) {
+    if (ready) {
       const int row = wrow0 + lane;
-      set_thresholds(row < rows_total ? row_max_of(a, (int64_t)h * a.q_rows_pad + row) : 0.0f, true);
+      float v = 0.0f;
+      if (row < rows_total) {
+        v = a.srmax[(int64_t)h * a.q_rows_pad + row];
+        if (a.keys1 || !own) v = row_key_value(__float_as_uint(v));
+      }
+      set_thresholds(v, own);
     } else {
       run_pass(std::integral_constant<int, 0>{}, 0, nall);
       set_thresholds(swept_max(), false);
@@ -1474,9 +1490,17 @@ static int exact_pass2_forced() {
   return e && e[0] == '1' ? 1 : 0;
 }
 
+// STA_SCORE_PIECES=n: every launch whose keys may be split takes n pieces a row group, as a grid of
+// several rounds does, for comparisons (0: the rule below)
+static int score_pieces_forced() {
+  const char* e = getenv("STA_SCORE_PIECES");
+  return e ? std::max(0, std::min(atoi(e), 1024)) : 0;
+}
+
 // How a launch splits its row groups' 64-key chunks over workgroups.
 struct ChunkSplit {
   int pieces, chunks;    // workgroups per row group, chunks per workgroup
+  bool rounds;           // split into more workgroups than the chip holds at once
 };
 
 // chunks of row group g of wg_rows rows
@@ -1501,7 +1525,11 @@ static ChunkSplit split_chunks(int H, int64_t q_pos_base, int64_t rows, int wg_r
   constexpr int CUS = 256;
   const int ng = (int)((rows + wg_rows - 1) / wg_rows);
   const int nall = (int)group_chunks(q_pos_base, rows, wg_rows, ng - 1);
-  ChunkSplit best{1, nall};
+  ChunkSplit best{1, nall, false};
+  if (const int n = score_pieces_forced()) {
+    const int c = (nall + n - 1) / n;
+    return ChunkSplit{(nall + c - 1) / c, c, n > 1};
+  }
   if ((int64_t)H * ng > 2 * CUS) return best;
   const double fixed = (waves == 8 ? 6.0 : 10.0) * 128 / D;
   const double load = (double)chunk_steps(H, q_pos_base, rows, wg_rows);
@@ -1514,7 +1542,7 @@ static ChunkSplit split_chunks(int H, int64_t q_pos_base, int64_t rows, int wg_r
     const double t = wgs <= CUS ? rounds : 0.5 * (rounds + (load + fixed * wgs) / CUS);
     if (t < t_best) {
       t_best = t;
-      best = ChunkSplit{(nall + c - 1) / c, c};
+      best = ChunkSplit{(nall + c - 1) / c, c, wgs > CUS};
     }
   }
   return best;
@@ -1557,6 +1585,9 @@ static hipError_t launch_score_t(const ScoreArgs& a0, hipStream_t st) {
     a.pieces = c.pieces;
     a.pchunks = c.chunks;
   };
+  // pass 2's keys are independent of each other, so any row group may be split (but its row counts)
+  const ChunkSplit whole{1, (int)(((int64_t)a.q_pos_base + rows + 63) / 64), false};
+  const ChunkSplit split2 = !RC && PQ != 6 ? split_chunks(a.H, a.q_pos_base, rows, 32 * RB * W2, D, W2) : whole;
   if (a.screened) {
     // Short calls take the key-split pass 1: up to 8192 (256-row group, 64-key chunk) steps, where
     // the four products of every score cost what the screen's candidate phase does (32 heads:
@@ -1566,17 +1597,24 @@ static hipError_t launch_score_t(const ScoreArgs& a0, hipStream_t st) {
     // concentrated scores on the three-product pass 2 (bf16, plain votes, 32 heads x 1000: 157 us a
     // call where the split pass 1 took 127, 8 x 5632: 354 against 394).
     a.keys1 = !a.fast6 && !screen_pass1_forced() && chunk_steps(a.H, a.q_pos_base, rows, 32 * RB * WS) <= 8192;
-    if (a.keys1) set_split(split_chunks(a.H, a.q_pos_base, rows, 32 * RB * WS, D, WS));
     // the same for every pass-2 epilogue: one instance per (D, T)
-    if (a.keys1)
-      hipLaunchKernelGGL((score_kernel<D, T, false, 0, RB, 2>), dim3(a.H * ng_s * a.pieces), dim3(64 * WS), 0, st, a);
-    else
+    if (!a.keys1) {
+      set_split(whole);
       hipLaunchKernelGGL((score_kernel<D, T, false, 0, RB, 1>), dim3(a.H * ng_s), dim3(64 * WS), 0, st, a);
+    }
   }
-  // pass 2's keys are independent of each other, so any row group may be split (but its row counts)
-  a.pieces = 1;
-  a.pchunks = (int)(((int64_t)a.q_pos_base + rows + 63) / 64);
-  if (!RC && PQ != 6) set_split(split_chunks(a.H, a.q_pos_base, rows, 32 * RB * W2, D, W2));
+  // The key-split sweep: pass 1 of the short calls, and of the row groups that the screen gave up
+  // where pass 2's pieces take several rounds (each piece would sweep its whole rows again; in one
+  // round that costs nothing).  With every score of a row tied, us a call, sweeping in each piece
+  // and once: fp32 1 head x 100000, D 64 21430 and 7280 (11300 with pass 2 whole), 16 x 8000, D 128
+  // 1814 and 1028 (1375), weighted 4 x 20000 3365 and 2114 (2293); the launch, which finds nothing
+  // to do on other inputs, takes 2-3 us.
+  a.swept = !a.keys1 && split2.rounds;
+  if (a.keys1 || a.swept) {
+    set_split(split_chunks(a.H, a.q_pos_base, rows, 32 * RB * WS, D, WS));
+    hipLaunchKernelGGL((score_kernel<D, T, false, 0, RB, 2>), dim3(a.H * ng_s * a.pieces), dim3(64 * WS), 0, st, a);
+  }
+  set_split(split2);
   if (a.fast6) {
     const hipError_t e = launch_score6(D, T, a, st);
     if (e != hipSuccess) return e;

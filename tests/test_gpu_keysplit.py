@@ -134,3 +134,53 @@ def test_concentrated_scores_keep_three_products(dt, tile, monkeypatch):
     (va, ma), (vb, mb) = got
     assert va.sum() > 10000
     assert np.array_equal(ma, mb) and np.array_equal(va, vb), f"{int((va != vb).sum())} vote entries differ"
+
+
+@pytest.mark.parametrize("H,Hkv,N,D,dt", [(2, 1, 1500, 128, torch.float32), (3, 3, 700, 64, torch.bfloat16),
+                                          (4, 2, 8300, 64, torch.float32)])
+@pytest.mark.parametrize("score", ["freq", "margin", "expmass"])
+@pytest.mark.parametrize("pieces", ["0", "1", "3", "7"])
+def test_groups_that_the_screen_gave_up(H, Hkv, N, D, dt, score, pieces, monkeypatch):
+    """The first half of one kv head's keys repeats one key: the screen gives up where rows see little
+    else, and the split pass 2 takes the maxima that a sweep of those row groups left.  The row-count
+    instance stays whole and sweeps inside.  (Whole plain votes sweep 512 rows where one half of them
+    was given up, the row-count instance 256: there all keys of the head are the same.)"""
+    import _sta_native as native
+    if dt != torch.float32 and score == "freq":
+        pytest.skip("whole instances have no fp6 pass 2")
+    say(f"screen gave up: H={H} Hkv={Hkv} N={N} D={D} {dt} {score} pieces={pieces}")
+    q, k, _, invf, tau = _inputs(H, Hkv, N, D, dt, 53)
+    k[:, 0, : N if score == "freq" and pieces in "01" else N // 2] = k[:, 0, :1]
+    monkeypatch.setenv("STA_SCREEN_PASS1", "1")
+    monkeypatch.setenv("STA_SCORE_PIECES", pieces)
+    got = []
+    for counts in (False, True):
+        r = native.select_vote(q, k, tau, invf, 0.0, 1.0, 1.0 / math.sqrt(D), 32, want_row_counts=counts, select_score=score)
+        torch.cuda.synchronize()
+        got.append([r[i].cpu().numpy() for i in range(len(r)) if i != 1])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b), f"{int((a != b).sum())} of {a.size} entries differ"
+
+
+def test_tied_scores_cost_one_sweep():
+    """100000 rows of one head, pass 2 in 17 pieces: a call whose scores all tie sweeps the maxima once
+    more, 1.4 times a call whose scores do not (3.3 times when every piece swept them)."""
+    import time
+    import _sta_native as native
+    from synthetic import base_inv_freq
+    N, D = 100000, 64
+    say("tied scores, 1 head x 100000")
+    g = torch.Generator(DEV).manual_seed(3)
+    q, k = (torch.randn(1, 1, N, D, generator=g, device=DEV) for _ in range(2))
+    invf = base_inv_freq(D, 10000.0).to(DEV)
+    best = []
+    for keys in (k, k[:, :, :1].repeat(1, 1, N, 1)):
+        t = []
+        for _ in range(4):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            native.select_vote(q, keys, torch.full((1,), 4.0), invf, 0.0, 1.0, 0.125, 64, want_row_counts=False)
+            torch.cuda.synchronize()
+            t.append(time.perf_counter() - t0)
+        best.append(min(t[1:]))
+    assert best[1] < 2.4 * best[0], f"{best[1] * 1e3:.2f} ms with ties, {best[0] * 1e3:.2f} without"
