@@ -74,9 +74,9 @@ struct ScoreArgs {
   int exact_pass1;        // 1: always run the three-product pass 1 sweep
   int screened;           // set by the launcher: the screen kernel ran before the pass-2 kernel
   float* srmax;           // (H, q_rows_pad) the screen's exact raw row maxima
-  int* sflags;            // (H, ngroups) the screen's fallback flags
+  int* sflags;            // (H, ngroups) the 256-row groups scored in three products in pass 1 too
   int keys1;              // set by the launcher: pass 1 ran as the key-split sweep, and srmax holds
-                          // order keys (row_key) instead of floats; sflags is not written
+                          // order keys (row_key) instead of floats
   int swept;              // set by the launcher: behind the screen, the key-split sweep left order keys
                           // in srmax for the row groups with sflags (without the screen: for all)
   int pieces, pchunks;    // set by the launcher, per launch: a row group's 64-key chunks are split

@@ -355,7 +355,8 @@ __global__ __launch_bounds__(1024) void norm_max_kernel(NormJob jq, NormJob jk) 
 // flag, for MODE 0, which runs pass 2 (and the three-product pass 1 where the screen fell back).
 // MODE 2 is the pass 1 of small calls: every score as the four products the screen takes for its
 // candidates (so the same maxima, bit for bit), the keys of a row group split over workgroups and
-// the rows' maxima merged by atomicMax.  The screen's candidate phase takes each wave 100 k cycles
+// the rows' maxima merged by atomicMax; over three products the row groups that it flags, and those
+// that the screen flagged.  The screen's candidate phase takes each wave 100 k cycles
 // however short its rows are, and one workgroup per 256 rows leaves most of the chip idle.
 // Waves per workgroup.  The screen: 4 (one per SIMD, two workgroups per CU).  Pass 2 with plain
 // votes: 8 (two per SIMD sharing each LDS chunk; each block's epilogue follows its own MFMAs and
@@ -425,9 +426,21 @@ void score_kernel(ScoreArgs a) {
   const int nall = (hi_max + CK - 1) / CK;
   const int nchunks = MODE == 1 ? nall : min(nall, c0 + a.pchunks);
   if (c0 >= nchunks) return;
-  // MODE 2 behind the screen: the row groups that it gave up
+  // the bound on a row's four-product scores' distance from its three-product ones
+  auto four_product_delta = [](float2 qn, float2 knm) {
+    return 1.001f * (qn.y * knm.y + 0x1p-15f * (qn.x + qn.y) * (knm.x + knm.y));
+  };
+  bool near = false;
   if constexpr (MODE == 2) {
+    // behind the screen: the row groups that it gave up
     if (!a.keys1 && a.screened && a.sflags[h * ngroups + g] == 0) return;
+    // Of a short call, the groups whose thresholds the cap at max - delta could move take three products
+    // in both passes, as where the screen gives up: a tau near 0, one key so far out that delta spans
+    // the head's scores, rows or keys that are not finite.  (1.05: the thresholds' rounding)
+    if (a.keys1 && active && wrow0 + lane < a.N) {
+      const float delta = four_product_delta(a.qnorm[(int64_t)h * a.q_rows_pad + wrow0 + lane], a.knorm_max[kvh]);
+      near = !(fabsf(a.tau[h]) > 1.05f * delta * a.sm_scale);
+    }
   }
   // chunks entirely below N whose keys are causal for every query of the workgroup
   const int nfull_all = min(min(nall, (a.q_pos_base + g * WG_ROWS + 1) / CK), a.N / CK);
@@ -1183,8 +1196,7 @@ void score_kernel(ScoreArgs a) {
     float x0 = ok ? min_arg_for(m - tau, a.sm_scale) : INFINITY;
     if (screened && ok && tau >= 0.0f) {
       const float2 qn = a.qnorm[(int64_t)h * a.q_rows_pad + grow];
-      const float delta = 1.001f * (qn.y * knm.y + 0x1p-15f * (qn.x + qn.y) * (knm.x + knm.y));
-      if (delta < INFINITY) x0 = fminf(x0, v - delta);   // no bound: rows or keys that are not finite
+      x0 = fminf(x0, v - four_product_delta(qn, knm));
     }
     if (a.row_max && ok) a.row_max[(int64_t)h * a.N + grow] = m;
     const float rf = WM == 1 ? m - tau : m;   // perquery.py:210, 215; exact_2.py:130, 135
@@ -1359,8 +1371,10 @@ void score_kernel(ScoreArgs a) {
     }
     return;
   } else if constexpr (MODE == 2) {
-    if (a.keys1) run_pass(std::integral_constant<int, 2>{}, c0, nchunks);
-    else run_pass(std::integral_constant<int, 0>{}, c0, nchunks);
+    const bool three = !a.keys1 || __syncthreads_or(near);
+    if (a.keys1 && piece == 0 && threadIdx.x == 0) a.sflags[h * ngroups + g] = three ? 1 : 0;
+    if (three) run_pass(std::integral_constant<int, 0>{}, c0, nchunks);
+    else run_pass(std::integral_constant<int, 2>{}, c0, nchunks);
     const float v = swept_max();
     if (active && wrow0 + lane < rows_total)
       atomicMax((uint32_t*)a.srmax + (int64_t)h * a.q_rows_pad + wrow0 + lane, row_key(v));
@@ -1369,14 +1383,14 @@ void score_kernel(ScoreArgs a) {
     // here where the screen fell back or is off
     // the screen's workgroups covering this one's rows (4 waves of 32 RB rows each)
     bool ready = a.keys1 || a.swept, own = a.screened;
-    if (!a.keys1 && a.screened) {
+    if (a.screened) {
       constexpr int SG = score_waves<false, 0, 1>() * 32 * RB;
       const int ng_s = (rows_total + SG - 1) / SG;
       bool all = true;
       for (int gs = g * WG_ROWS / SG; gs < min((g + 1) * WG_ROWS / SG, ng_s); ++gs)
         all = all && a.sflags[h * ng_s + gs] == 0;
       ready = ready || all;
-      own = active && a.sflags[h * ng_s + wrow0 / SG] == 0;   // this wave's rows kept the screen's maxima
+      own = active && a.sflags[h * ng_s + wrow0 / SG] == 0;   // this wave's rows have four-product maxima
     }
     if (ready) {
       const int row = wrow0 + lane;

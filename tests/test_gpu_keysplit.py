@@ -184,3 +184,33 @@ def test_tied_scores_cost_one_sweep():
             t.append(time.perf_counter() - t0)
         best.append(min(t[1:]))
     assert best[1] < 2.4 * best[0], f"{best[1] * 1e3:.2f} ms with ties, {best[0] * 1e3:.2f} without"
+
+
+@pytest.mark.parametrize("H,Hkv,N,D", [(2, 2, 1500, 128), (4, 2, 700, 64)])
+@pytest.mark.parametrize("tau", [0.0, 4.0])
+@pytest.mark.parametrize("far", [1e6, float("inf")])
+def test_one_key_far_out(H, Hkv, N, D, tau, far):
+    """The last key a million times as long as the others, or with an infinite element: the rows that
+    do not see it keep what the oracle keeps without it, and each of them its best key (the bound on
+    the four-product maxima spans all of the head's scores, or is not finite)."""
+    import _sta_native as native
+    from oracle import sta_oracle as orc
+    from parity_helpers import BAND, np_of
+    say(f"one key far out: H={H} Hkv={Hkv} N={N} D={D} x{far} tau={tau}")
+    q, k, _, invf, _ = _inputs(H, Hkv, N, D, torch.float32, 43)
+    taus = torch.full((H,), tau)
+    qn, odt = np_of(q[0])
+    kn, _ = np_of(k[0])
+    sm = 1.0 / math.sqrt(D)
+    a = orc.select_vote(qn, kn, odt, taus.numpy(), invf.cpu().numpy(), 0.5, 1.0, sm, 32, 0, band_eps=BAND, want_band=True)
+    if far < float("inf"):
+        k[:, 0, N - 1] *= far
+    else:
+        k[:, 0, N - 1, 5] = far
+    votes, _, rm = native.select_vote(q, k, taus, invf, 0.5, 1.0, sm, 32, want_row_counts=False)
+    torch.cuda.synchronize()
+    votes, rm = votes.cpu().numpy().astype(np.int64), rm.cpu().numpy()
+    assert np.abs(rm - a["row_max"])[:, : N - 1].max() < 1e-4
+    nt = (N - 1) // 32
+    assert (np.abs(votes - a["votes"])[:, :nt] <= a["band"][:, :nt]).all()
+    assert (votes[:, :nt].sum(-1) >= 32).all()
