@@ -1176,8 +1176,13 @@ class DecodePlan:
                "sta_decode_scores")
         return out
 
+    def _check_sets(self):
+        if "idx" not in self.out:
+            raise RuntimeError("a plan with sets=False returns no sets")
+
     def build_sets(self, scores):
         """Selection alone from scores (H, Q, M) fp32 into idx / newpos_k / newpos_q / set_size."""
+        self._check_sets()
         _check(lib().sta_decode_build_sets(ctypes.byref(self.args), _ptr(scores), _stream(self.device)),
                "sta_decode_build_sets")
         return self.out
@@ -1187,6 +1192,7 @@ class DecodePlan:
         """The chunk rule (_decode_build_sets_chunk, chunked.py:411-489) from scores (H, Q, M) fp32
         into idx / newpos_k / newpos_q / set_size (the kept count); passers_kept and usize (H, Q)
         int32 receive the threshold passers among the kept keys and in all, when given."""
+        self._check_sets()
         cp = _chunk_params(chunk_size, n_chunk, chunk_agg, passers_kept)
         a = self.args
         saved = a.usize

@@ -386,3 +386,16 @@ def test_decode_without_set_arrays(rule, H, Hkv, Q, M, km):
         assert torch.equal(out, r["out"])
     for name in stats:
         assert torch.equal(stats[name], r[name])
+
+
+def test_plan_without_set_arrays_builds_no_sets():
+    """The sets lie where no caller sees them: asking for them is an error, not a dict without them."""
+    import _sta_native as native
+    H, M = 2, 200
+    q, k = torch.randn(H, 1, 64, device=DEV), torch.randn(H, M, 64, device=DEV)
+    plan = native.DecodePlan(q, k, k, torch.ones(H), torch.ones(32), M - 1, k_max=64, sets=False)
+    scores = torch.zeros(H, 1, M, device=DEV)
+    with pytest.raises(RuntimeError, match="sets=False"):
+        plan.build_sets(scores)
+    with pytest.raises(RuntimeError, match="sets=False"):
+        plan.build_sets_chunk(scores, 32, 2)
