@@ -15,7 +15,7 @@
 //
 // Launches: the scores (one workgroup = one kv head x 256 keys, all heads of the group; scores
 // plus each block's max and sum of exp), dca_dec_pv_kernel (one workgroup = one kv head x 256
-// keys, all heads of the group: global max and sum from the block partials, weights, partial
+// keys, a few heads of the group: global max and sum from the block partials, weights, partial
 // P.V), and dca_dec_combine_kernel (sum of the partials, rounded to the dtype).  16-bit caches
 // take dca_dec_score16_kernel, which rotates the queries itself and scores on the matrix cores;
 // fp32 caches take dca_dec_qrot_kernel (the three query variants of every head) and
@@ -313,16 +313,16 @@ __global__ __launch_bounds__(DCA_DEC_BK) void dca_dec_score16_kernel(DcaDecArgs 
 }
 
 // ------------------------------------------------------------------------------------------
-// softmax weights and partial P.V of the heads of kv head g over the keys [256 b, 256 b + 256).
+// softmax weights and partial P.V of GP heads of kv head g (the last workgroup of a group: those
+// left) over the keys [256 b, 256 b + 256).
 //
-// HBM-bound: every value row is read once, for all heads of its group (GP: the group rounded up to
-// a power of two), D / 8 lanes a row in 16-byte pieces.  The first PF rows of a lane are requested
+// HBM-bound: every value row is read once for GP heads, D / 8 lanes a row in 16-byte pieces.  The first PF rows of a lane are requested
 // before the block partials are reduced and the weights taken, so they arrive meanwhile.  65535
 // keys, 32 query / 8 kv heads, D 128, bf16: 29.5 us, 4.6 TB/s (one workgroup a query head with
 // 2-byte loads: 220 us; all 16 rows of a lane in flight, two workgroups a CU: 50 us).
 // ------------------------------------------------------------------------------------------
 template <int DT, int D, int GP>
-__global__ __launch_bounds__(DCA_DEC_BK, DT != DT_F32 && GP <= 4 ? 4 : 1) void dca_dec_pv_kernel(DcaDecArgs a) {
+__global__ __launch_bounds__(DCA_DEC_BK, DT != DT_F32 ? 4 : 1) void dca_dec_pv_kernel(DcaDecArgs a) {
 #pragma clang fp contract(off)
   constexpr int LPR = D / 8;                   // lanes per row
   constexpr int RPS = DCA_DEC_BK / LPR;        // rows per step of the workgroup
@@ -337,6 +337,8 @@ __global__ __launch_bounds__(DCA_DEC_BK, DT != DT_F32 && GP <= 4 ? 4 : 1) void d
   const int tid = threadIdx.x;
   const int lane = tid & 63, wid = tid >> 6;
   const int G = a.H / a.Hkv;
+  const int h0 = g * G + blockIdx.z * GP;      // this workgroup's heads: [h0, h0 + nh)
+  const int nh = min(GP, G - (int)blockIdx.z * GP);
   const int c = tid % LPR, row = tid / LPR;
   const int64_t vb = (int64_t)g * a.v_head_stride + 8 * c;
   Raw8<DT> v[PF];
@@ -351,11 +353,11 @@ __global__ __launch_bounds__(DCA_DEC_BK, DT != DT_F32 && GP <= 4 ? 4 : 1) void d
   const int j = blk * DCA_DEC_BK + tid;
   float sc[GP];
 #pragma unroll
-  for (int u = 0; u < GP; ++u) sc[u] = u < G && j < a.M ? a.scores[(int64_t)(g * G + u) * a.M + j] : 0.0f;
+  for (int u = 0; u < GP; ++u) sc[u] = u < nh && j < a.M ? a.scores[(int64_t)(h0 + u) * a.M + j] : 0.0f;
   // the global max and the sum of exp(s - max) of each head from the blocks' partials, a wave a head
-  for (int u = wid; u < G; u += W) {
-    const float* pm = a.pmax + (int64_t)(g * G + u) * a.nb;
-    const float* ps = a.psum + (int64_t)(g * G + u) * a.nb;
+  for (int u = wid; u < nh; u += W) {
+    const float* pm = a.pmax + (int64_t)(h0 + u) * a.nb;
+    const float* ps = a.psum + (int64_t)(h0 + u) * a.nb;
     constexpr int R = 4;                       // partials a lane holds: 256 blocks, 65536 keys
     float pr[R], sr[R], m = -INFINITY;
 #pragma unroll
@@ -383,7 +385,7 @@ __global__ __launch_bounds__(DCA_DEC_BK, DT != DT_F32 && GP <= 4 ? 4 : 1) void d
 #pragma unroll
   for (int u = 0; u < GP; ++u) {
     float p = 0.0f;
-    if (u < G && j < a.M) p = round_dt<DT>(opaque_f32(expf(sc[u] - gm[u]) / gl[u]));
+    if (u < nh && j < a.M) p = round_dt<DT>(opaque_f32(expf(sc[u] - gm[u]) / gl[u]));
     pS[tid * GP + u] = p;
   }
   __syncthreads();
@@ -419,12 +421,12 @@ __global__ __launch_bounds__(DCA_DEC_BK, DT != DT_F32 && GP <= 4 ? 4 : 1) void d
       if (lane < LPR) red[wid][u][8 * c + e] = x;
     }
   __syncthreads();
-  for (int i = tid; i < G * D; i += DCA_DEC_BK) {
+  for (int i = tid; i < nh * D; i += DCA_DEC_BK) {
     const int u = i / D, d = i % D;
     float s = red[0][u][d];
 #pragma unroll
     for (int w = 1; w < W; ++w) s += red[w][u][d];
-    a.part[((int64_t)(g * G + u) * a.nb + blk) * D + d] = s;
+    a.part[((int64_t)(h0 + u) * a.nb + blk) * D + d] = s;
   }
 }
 
@@ -494,13 +496,18 @@ static hipError_t launch_dca_decode_t(const DcaDecArgs& a, hipStream_t st) {
   hipError_t e = launch_dca_scores_t<DT, D>(a, st);
   if (e != hipSuccess) return e;
   const int G = a.H / a.Hkv;
-  const dim3 grid(a.Hkv, a.nb);
-#define STA_PV(GP_) hipLaunchKernelGGL((dca_dec_pv_kernel<DT, D, GP_>), grid, dim3(DCA_DEC_BK), 0, st, a)
-  if (G == 1) STA_PV(1);
+  // Heads per P.V workgroup: four read a value row's bytes once and stay short; more unrolled code
+  // costs a small call its fetch.  fp32, one head a workgroup below 1024 of them (16 heads / 1 kv head
+  // x 100, D 64: 36.4 us a call, four 39.6, all sixteen 54.1), eight at D 128 from 4096 (32 / 4 x
+  // 65535: 92 us, four 104; 16-bit 52.6 and 50.5).
+  const int64_t wgs = (int64_t)a.H * a.nb;
+  int gp = 4;
+  if (DT == DT_F32) gp = wgs < 1024 ? 1 : (D == 128 && wgs >= 4096 ? 8 : 4);
+#define STA_PV(GP_) hipLaunchKernelGGL((dca_dec_pv_kernel<DT, D, GP_>), dim3(a.Hkv, a.nb, (G + GP_ - 1) / GP_), dim3(DCA_DEC_BK), 0, st, a)
+  if (gp == 1 || G == 1) STA_PV(1);
   else if (G == 2) STA_PV(2);
-  else if (G <= 4) STA_PV(4);
-  else if (G <= 8) STA_PV(8);
-  else STA_PV(16);
+  else if (gp == 4 || G <= 4) STA_PV(4);
+  else if constexpr (DT == DT_F32 && D == 128) STA_PV(8);
 #undef STA_PV
   if ((e = hipGetLastError()) != hipSuccess) return e;
   hipLaunchKernelGGL((dca_dec_combine_kernel<DT, D>), dim3(a.H, D / 32), dim3(512), 0, st, a);

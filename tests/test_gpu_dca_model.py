@@ -142,6 +142,52 @@ def test_decode_group_sizes_and_block_edges(dt, D, H, Hkv):
         ulp_close(out.float().cpu().numpy(), ref, dt, f"groups M={M}", vmax=float(v.float().abs().max()))
 
 
+@pytest.mark.parametrize("dt,D,H,Hkv,M", [
+    # one head a P.V workgroup (fp32, below 1024 of them), four (the last workgroup of a group
+    # with one, two and all of them), eight (fp32, D 128, from 4096; the last with one and four)
+    (torch.float32, 64, 16, 1, 100), (torch.float32, 128, 32, 2, 7936), (torch.float32, 128, 32, 2, 7937),
+    (torch.float32, 64, 12, 1, 22000), (torch.bfloat16, 128, 5, 1, 700), (torch.float16, 64, 28, 2, 3000),
+    (torch.bfloat16, 64, 32, 4, 513), (torch.float32, 128, 18, 2, 58300), (torch.float32, 128, 24, 2, 43700),
+])
+def test_decode_group_head_equals_the_head_alone(dt, D, H, Hkv, M):
+    """A head's output does not depend on the heads that share its workgroups: bit for bit the call
+    with its query and its kv head alone."""
+    import _sta_native as native
+    say(f"dca decode, heads alone: {dt} D={D} H={H} Hkv={Hkv} M={M}")
+    g = torch.Generator(DEV).manual_seed(59 + M)
+    q = torch.randn(H, D, generator=g, device=DEV).to(dt)
+    k, v = (torch.randn(Hkv, M, D, generator=g, device=DEV).to(dt) for _ in range(2))
+    out = native.dca_decode(q, k, v, _inv_freq(D), 130, 33, 1.0254)
+    for h in range(H):
+        hk = h // (H // Hkv)
+        one = native.dca_decode(q[h:h + 1], k[hk:hk + 1], v[hk:hk + 1], _inv_freq(D), 130, 33, 1.0254)
+        assert torch.equal(one[0], out[h]), f"head {h}"
+
+
+def test_decode_wide_group_over_a_short_cache():
+    """Sixteen heads of one kv head over 100 fp32 keys: 1.95 times one head's call (2.9 times when one
+    P.V workgroup took all sixteen)."""
+    import time
+    import _sta_native as native
+    say("dca decode, 16 heads and 1 over 100 keys")
+    g = torch.Generator(DEV).manual_seed(61)
+    q = torch.randn(16, 64, generator=g, device=DEV)
+    k, v = (torch.randn(1, 100, 64, generator=g, device=DEV) for _ in range(2))
+    inv = _inv_freq(64).to(DEV)
+    best = []
+    for heads in (1, 16):
+        t = []
+        for _ in range(8):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(100):
+                native.dca_decode(q[:heads], k, v, inv, 130, 33, 1.0254)
+            torch.cuda.synchronize()
+            t.append((time.perf_counter() - t0) / 100)
+        best.append(min(t))
+    assert best[1] < 2.4 * best[0], f"{best[1] * 1e6:.1f} us, one head {best[0] * 1e6:.1f}"
+
+
 def test_decode_matches_reference_goldens():
     import _sta_native as native
     g = np.load(os.path.join(GOLD, "dca_decode_golden.npz"), allow_pickle=False)
