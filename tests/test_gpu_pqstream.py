@@ -381,3 +381,33 @@ def test_stream_workgroup_sizes_and_mask_edges(dt, H, N, D, block_n):
         err = np.abs(r["out"][h:h + 1].float().cpu().numpy() - out)
         tol = 1e-4 if dt == torch.float32 else 2e-2 + 1e-2 * np.abs(out)
         assert np.all(err <= tol), f"head {h}: {err.max():.3e}"
+
+
+@pytest.mark.parametrize("dt,block_n", [(torch.float32, 32), (torch.bfloat16, 32), (torch.bfloat16, 64), (torch.float16, 32)])
+@pytest.mark.parametrize("fused", ["unfused", "fused"])
+def test_stream_best_key_weighs_one(dt, block_n, fused):
+    """Rows of two keys: one of weight w, met first, then the best key.  The best key's weight is 1, exact
+    in every type, so the output is off by w's rounding (2^-9 in bf16, 2^-12 in fp16, 2^-17 for fp32's
+    pair) and its own alone.  Scores gap 2 .. 5.4 apart, no rotation; the other keys weigh e^-40."""
+    import _sta_native as native
+    H, N, D = 2, 400, 64
+    say(f"stream, best key last: {dt} block_n={block_n} {fused}")
+    g = torch.Generator().manual_seed(67)
+    gap = torch.linspace(2.0, 5.4, N).to(dt)
+    q, k = torch.zeros(1, H, N, D), torch.zeros(1, H, N, D)
+    q[..., 0] = gap.float()                                   # sm_scale 1: scores gap, 0 and -20 gap
+    k[..., 0] = -20.0
+    k[:, :, 0, 0], k[:, :, 70, 0] = 1.0, 0.0
+    v = torch.randn(1, H, N, D, generator=g).to(torch.bfloat16).to(dt)   # exact in every type's operands
+    zero = torch.zeros(D // 2)
+    r = native.pqstream_attention(q.to(dt).to(DEV), k.to(dt).to(DEV), v.to(DEV), torch.full((H,), 7.0), zero, zero, 1.0, 1.0,
+                                  sm_scale=1.0, block_n=block_n, fused=fused)
+    torch.cuda.synchronize()
+    out = r["out"].cpu()[:, 128:].double()                    # rows whose blocks end past both keys
+    w = torch.exp(-gap.double())[128:, None]
+    a, b = v[0, :, :1].double(), v[0, :, 70:71].double()
+    ref = (a + w * b) / (1 + w)
+    eps = {torch.float32: 2.0 ** -17, torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}[dt]
+    e = w * eps * b.abs() + 2.0 ** -20 * (a.abs() + b.abs())   # fp32 exp2 and sums
+    assert bool(((out >= (ref - e).to(dt).double()) & (out <= (ref + e).to(dt).double())).all()), \
+        f"{float(((out - ref).abs() / ref.abs().clamp_min(0.1)).max()):.2e}"
