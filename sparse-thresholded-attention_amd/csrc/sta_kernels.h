@@ -89,7 +89,6 @@ struct ScoreArgs {
   const float2* qnorm_max;// (H,) maxima of (||q_hi||, ||q_lo||)
   const uint64_t* q6;     // fp6 planes / scales / error norms of the Q and K fragments
   const uint32_t* q6sc;
-  const float2* q6dn;     // (H, q_rows_pad) per row
   const float2* q6dmax;   // (H,)
   const uint64_t* k6;
   const uint32_t* k6sc;
@@ -391,8 +390,9 @@ __device__ __forceinline__ void score_workgroup(int bid, int H, int ngroups, int
 // Whether the fp6 pass-2 kernel (sta_score6.hip) serves workgroup g (wg_rows query rows) of
 // head h in the plain pass 2; the three-product kernel then skips it.  It does when the launcher
 // enabled it, the screened pass 1 resolved every row of the workgroup (its 256-row workgroups
-// raised no fallback flag) and the head's fp6 error estimate stays within the limit.  Both
-// kernels evaluate this one function on the same inputs.
+// raised no fallback flag), the head's fp6 error estimate stays within the limit, and tau exceeds
+// the bound on that error: a row's best key then passes (tau > 0) or no key does (tau < 0),
+// whatever the rounding.  Both kernels evaluate this one function on the same inputs.
 __device__ inline bool fast6_serves(const ScoreArgs& a, int h, int g, int D, int wg_rows) {
   if (!a.fast6) return false;
   const int rows_total = a.q_rows_pad;
@@ -403,7 +403,8 @@ __device__ inline bool fast6_serves(const ScoreArgs& a, int h, int g, int D, int
   const int kvh = h / (a.H / a.Hkv);
   const float2 qn = a.qnorm_max[h], kn = a.knorm_max[kvh], qd = a.q6dmax[h], kd = a.k6dmax[kvh];
   const float sg = fast6_sigma(qn.x, qn.y, qd.x, qd.y, kn.x, kn.y, kd.x, kd.y, a.sm_scale, D);
-  return sg <= FAST6_SIGMA_LIMIT;
+  const float delta = fast6_delta(qn.x, qn.y, qd.x, qd.y, kn.x, kn.y, kd.x, kd.y);
+  return sg <= FAST6_SIGMA_LIMIT && fabsf(a.tau[h]) > 1.05f * delta * a.sm_scale;   // 1.05: x0's rounding
 }
 
 // One side of the selection-geometry RoPE pre-kernel: `heads` heads of N rows (positions pos_base

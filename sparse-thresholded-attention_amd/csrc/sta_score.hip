@@ -1589,7 +1589,6 @@ static hipError_t launch_score_t(const ScoreArgs& a0, hipStream_t st) {
     a.qnorm_max = frag_norm_max(a.qfrag, a.H, a.q_rows_pad, D);
     a.q6 = frag6_planes(a.qfrag, a.H, a.q_rows_pad, D);
     a.q6sc = frag6_scales(a.qfrag, a.H, a.q_rows_pad, D);
-    a.q6dn = frag6_dnorms(a.qfrag, a.H, a.q_rows_pad, D);
     a.q6dmax = frag6_dnorm_max(a.qfrag, a.H, a.q_rows_pad, D);
     a.k6 = frag6_planes(a.kfrag, a.Hkv, a.k_rows_pad, D);
     a.k6sc = frag6_scales(a.kfrag, a.Hkv, a.k_rows_pad, D);

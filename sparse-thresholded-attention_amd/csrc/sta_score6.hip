@@ -99,29 +99,24 @@ __global__ __launch_bounds__(512, 1) void score6_kernel(ScoreArgs a) {
   uint8_t* vrow = a.votes + ((int64_t)h * a.nt + wrow0 / T) * a.votes_stride;
   auto tile_ok = [&](int j) { return wrow0 + j * T < rows_total; };
 
-  // ---- keep thresholds x0 on the raw dot from the screen's exact row maxima.  For tau >= 0 the
-  // threshold is capped at max - delta (delta bounds the fp6 score's distance from the screen's
-  // exact dot, sta_fp6.h: fast6_delta), so a row's best key keeps its vote, as in the reference
-  // whose two passes share one dot.  Row block 0's accumulators start from -x0 (held in the
-  // AGPRs beside the Q operands), so its products accumulate s - x0 and the keep test is the
-  // accumulator's sign (that rounding, ~1e-6 of the score, is far inside the correction's error);
-  // row block 1 keeps x0 in VGPRs and subtracts it (the register file holds one set of each).
+  // ---- keep thresholds x0 on the raw dot from the screen's exact row maxima.  They lie further from
+  // the maxima than any fp6 score from the screen's exact dot (fast6_serves), so a row's best key
+  // keeps its vote, as in the reference whose two passes share one dot.  Row block 0's accumulators
+  // start from -x0 (held in the AGPRs beside the Q operands), so its products accumulate s - x0 and
+  // the keep test is the accumulator's sign (that rounding, ~1e-6 of the score, is far inside the
+  // correction's error); row block 1 keeps x0 in VGPRs and subtracts it (the register file holds one
+  // set of each).
   float* xs = (float*)&lds[(c0 + NBUF - 1) % NBUF][0] + wave * 64;
   {
     // one row per lane, read back into the lane's 32 row slots (min_arg_for's division and
     // nextafter steps on every slot cost each wave 32 times as many)
     static_assert(32 * RB == 64, "one wave row per lane");
-    const float2 knm = a.knorm_max[kvh], kd = a.k6dmax[kvh];
     const int row = wrow0 + lane;
     const bool ok = active && row < a.N;       // padded rows never vote (exact_2.py:121)
     const int64_t ri = (int64_t)h * a.q_rows_pad + (row < rows_total ? row : 0);
     const float v = a.srmax[ri];
     const float m = v * a.sm_scale;            // fl(max * c) == max of fl(s * c) for c > 0
-    float x = ok ? min_arg_for(m - tau, a.sm_scale) : INFINITY;
-    if (ok && tau >= 0.0f) {
-      const float2 qn = a.qnorm[ri], qd = a.q6dn[ri];
-      x = fminf(x, v - fast6_delta(qn.x, qn.y, qd.x, qd.y, knm.x, knm.y, kd.x, kd.y));
-    }
+    const float x = ok ? min_arg_for(m - tau, a.sm_scale) : INFINITY;
     if (a.row_max && ok) a.row_max[(int64_t)h * a.N + row] = m;
     // through the last chunk buffer, which no copy reaches before the sweep's first barrier
     xs[lane] = -x;

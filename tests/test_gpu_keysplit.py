@@ -214,3 +214,45 @@ def test_one_key_far_out(H, Hkv, N, D, tau, far):
     nt = (N - 1) // 32
     assert (np.abs(votes - a["votes"])[:, :nt] <= a["band"][:, :nt]).all()
     assert (votes[:, :nt].sum(-1) >= 32).all()
+
+
+def _oracle(q, k, tau, invf, ps, tile):
+    from oracle import sta_oracle as orc
+    from parity_helpers import BAND, np_of
+    qn, dt = np_of(q[0])
+    kn, _ = np_of(k[0])
+    return orc.select_vote(qn, kn, dt, tau.numpy(), invf.cpu().numpy(), ps, 1.0, 1.0 / math.sqrt(q.shape[-1]), tile,
+                           band_eps=BAND, want_band=True)
+
+
+def _votes(q, k, tau, invf, ps, tile, counts):
+    import _sta_native as native
+    votes, rc, rm = native.select_vote(q, k, tau, invf, ps, 1.0, 1.0 / math.sqrt(q.shape[-1]), tile, want_row_counts=counts)
+    torch.cuda.synchronize()
+    return votes.cpu().numpy().astype(np.int64), rc.cpu().numpy() if counts else None, rm.cpu().numpy()
+
+
+PATHS = pytest.mark.parametrize("screen,pieces", [("0", "0"), ("0", "4"), ("1", "0"), ("1", "4")])
+KINDS = pytest.mark.parametrize("dt,counts", [(torch.bfloat16, False), (torch.bfloat16, True), (torch.float32, False)])
+
+
+@PATHS
+@KINDS
+def test_tau_zero_and_below(dt, counts, screen, pieces, monkeypatch):
+    """tau = 0: each row keeps its best key and none beyond the band; tau < 0: no key."""
+    H, N, D = 2, 2000, 128
+    say(f"tau 0 and below: {dt} counts={counts} screen={screen} pieces={pieces}")
+    q, k, _, invf, _ = _inputs(H, H, N, D, dt, 12)
+    monkeypatch.setenv("STA_SCREEN_PASS1", screen)
+    monkeypatch.setenv("STA_SCORE_PIECES", pieces)
+    tau = torch.zeros(H)
+    a = _oracle(q, k, tau, invf, 0.5, 64)
+    votes, rc, _ = _votes(q, k, tau, invf, 0.5, 64, counts)
+    assert (np.abs(votes - a["votes"]) <= a["band"]).all()
+    rows = np.minimum(64, N - 64 * np.arange(votes.shape[1]))
+    assert (votes.sum(-1) >= rows).all()
+    if counts:
+        assert (rc >= 1).all()
+    for low in (-0.5, -3.0):
+        votes, rc, _ = _votes(q, k, torch.full((H,), low), invf, 0.5, 64, counts)
+        assert votes.sum() == 0 and (not counts or rc.sum() == 0), low
