@@ -216,6 +216,31 @@ def test_one_key_far_out(H, Hkv, N, D, tau, far):
     assert (votes[:, :nt].sum(-1) >= 32).all()
 
 
+@pytest.mark.parametrize("H,Hkv,N,D,dt", [(2, 1, 65, 128, torch.float16), (3, 3, 700, 64, torch.float32),
+                                          (8, 2, 1601, 128, torch.bfloat16)])
+def test_forced_pieces_match_whole_groups(H, Hkv, N, D, dt, monkeypatch):
+    """Plain and weighted votes and per-query bits in 2, 5 and more pieces than chunks against one piece:
+    the sizes above split or not as the cost rule has it, here they do."""
+    import _sta_native as native
+    say(f"forced pieces: H={H} Hkv={Hkv} N={N} D={D} {dt}")
+    q, k, v, invf, tau = _inputs(H, Hkv, N, D, dt, 71)
+    sm = 1.0 / math.sqrt(D)
+    got = []
+    for pieces in ("1", "2", "5", "64"):
+        monkeypatch.setenv("STA_SCORE_PIECES", pieces)
+        out = []
+        for score in ("freq", "margin", "expmass"):
+            r = native.select_vote(q, k, tau, invf, 0.5, 1.0, sm, 32, want_row_counts=False, select_score=score)
+            out += [x.clone() for x in r if x is not None]
+        p = native.PqPlan(q, k, v, tau, invf, invf, 0.5, 1.0, k_max=512, want_votes=True, want_row_max=True).run()
+        out += [p[name].clone() for name in ("row_max", "votes", "bits", "wvotes", "out")]
+        torch.cuda.synchronize()
+        got.append(out)
+    for other in got[1:]:
+        for i, (a, b) in enumerate(zip(got[0], other)):
+            assert torch.equal(a, b), f"output {i}: {int((a != b).sum())} of {a.numel()} entries differ"
+
+
 def _oracle(q, k, tau, invf, ps, tile):
     from oracle import sta_oracle as orc
     from parity_helpers import BAND, np_of
@@ -238,6 +263,27 @@ KINDS = pytest.mark.parametrize("dt,counts", [(torch.bfloat16, False), (torch.bf
 
 @PATHS
 @KINDS
+def test_tied_scores(dt, counts, screen, pieces, monkeypatch):
+    """One key repeated, and zero query rows, on the short calls' pass 1 and behind the screen, with and
+    without row counts: maxima and votes of the oracle."""
+    H, N, D = 2, 1500, 128
+    say(f"tied scores: {dt} counts={counts} screen={screen} pieces={pieces}")
+    g = torch.Generator().manual_seed(5)
+    q, k = (torch.randn(1, H, N, D, generator=g) for _ in range(2))
+    q[:, :, 300:700] = 0.0
+    k[:, 0] = k[:, 0, :1]
+    q, k = q.to(dt).to(DEV), k.to(dt).to(DEV)
+    invf, tau = _inputs(H, H, 1, D, dt, 1)[3], torch.full((H,), 5.0)
+    a = _oracle(q, k, tau, invf, 0.0, 64)
+    monkeypatch.setenv("STA_SCREEN_PASS1", screen)
+    monkeypatch.setenv("STA_SCORE_PIECES", pieces)
+    votes, _, rm = _votes(q, k, tau, invf, 0.0, 64, counts)
+    assert np.abs(rm - a["row_max"]).max() < 1e-4
+    assert (np.abs(votes - a["votes"]) <= a["band"]).all()
+
+
+@PATHS
+@KINDS
 def test_tau_zero_and_below(dt, counts, screen, pieces, monkeypatch):
     """tau = 0: each row keeps its best key and none beyond the band; tau < 0: no key."""
     H, N, D = 2, 2000, 128
@@ -256,3 +302,27 @@ def test_tau_zero_and_below(dt, counts, screen, pieces, monkeypatch):
     for low in (-0.5, -3.0):
         votes, rc, _ = _votes(q, k, torch.full((H,), low), invf, 0.5, 64, counts)
         assert votes.sum() == 0 and (not counts or rc.sum() == 0), low
+
+
+@PATHS
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("tau", [0.0, 4.0])
+def test_finite_rows_beside_others(dt, tau, screen, pieces, monkeypatch):
+    """An infinite and a NaN query row and a NaN key: tiles without such a row, and rows before that
+    key, have the votes that the oracle gives them on finite inputs, and a key for every row."""
+    H, N, D, tile = 3, 700, 128, 32
+    say(f"rows and keys that are not finite: {dt} tau={tau} screen={screen} pieces={pieces}")
+    q, k, _, invf, _ = _inputs(H, H, N, D, dt, 41)
+    taus = torch.full((H,), tau)
+    a = _oracle(q, k, taus, invf, 0.5, tile)
+    q[0, 0, 100] = float("inf")
+    q[0, 2, 200, 7] = float("nan")
+    k[0, 1, 300, 5] = float("nan")
+    monkeypatch.setenv("STA_SCREEN_PASS1", screen)
+    monkeypatch.setenv("STA_SCORE_PIECES", pieces)
+    votes, _, _ = _votes(q, k, taus, invf, 0.5, tile, False)
+    ok = np.ones(votes.shape[:2], bool)
+    ok[0, 100 // tile] = ok[2, 200 // tile] = ok[1, 300 // tile:] = False
+    rows = np.minimum(tile, N - tile * np.arange(votes.shape[1]))
+    assert (np.abs(votes - a["votes"])[ok] <= a["band"][ok]).all()
+    assert (votes.sum(-1) >= rows)[ok].all()
