@@ -948,7 +948,13 @@ void score_kernel(ScoreArgs a) {
       rowbest[r] = 0u;
       rowcnt[r] = 0;
     }
+    // a row whose cap at max - delta could move its threshold by more than the set contract's band of
+    // 1e-3 (long rows, one key far out) sends the workgroup to the three-product sweep as well
     bool amb = false;
+    if (active && wrow0 + lane < a.N) {
+      const float loose = four_product_delta(a.qnorm[(int64_t)h * a.q_rows_pad + wrow0 + lane], kn) * a.sm_scale;
+      amb = !(loose <= 1e-3f || fabsf(tau) > 1.05f * loose);
+    }
     __syncthreads();
     float thr[RB][16];
     const int col = lane & 31;

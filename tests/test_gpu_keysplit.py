@@ -326,3 +326,38 @@ def test_finite_rows_beside_others(dt, tau, screen, pieces, monkeypatch):
     rows = np.minimum(tile, N - tile * np.arange(votes.shape[1]))
     assert (np.abs(votes - a["votes"])[ok] <= a["band"][ok]).all()
     assert (votes.sum(-1) >= rows)[ok].all()
+
+
+@PATHS
+@KINDS
+def test_tau_zero_with_long_rows(dt, counts, screen, pieces, monkeypatch):
+    """Rows four times as long: the bound on the four-product maxima exceeds the band, yet no key beyond
+    the band of a row's best key passes at tau = 0."""
+    H, N, D = 2, 1500, 128
+    say(f"tau 0, long rows: {dt} counts={counts} screen={screen} pieces={pieces}")
+    q, k, _, invf, _ = _inputs(H, H, N, D, dt, 13)
+    q, k = (4 * q.float()).to(dt), (4 * k.float()).to(dt)
+    tau = torch.zeros(H)
+    a = _oracle(q, k, tau, invf, 0.5, 64)
+    monkeypatch.setenv("STA_SCREEN_PASS1", screen)
+    monkeypatch.setenv("STA_SCORE_PIECES", pieces)
+    votes, _, _ = _votes(q, k, tau, invf, 0.5, 64, counts)
+    assert (np.abs(votes - a["votes"]) <= a["band"]).all()
+    rows = np.minimum(64, N - 64 * np.arange(votes.shape[1]))
+    assert (votes.sum(-1) >= rows).all()
+
+
+@pytest.mark.parametrize("N", [40, 700])
+@pytest.mark.parametrize("screen", ["0", "1"])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_one_key_far_out_of_few(N, screen, dt, monkeypatch):
+    """The same with so few keys that the screen scores all of them: every row keeps the oracle's."""
+    H, D = 2, 128
+    say(f"one key far out of {N}: {dt} screen={screen}")
+    q, k, _, invf, tau = _inputs(H, H, N, D, dt, 43)
+    a = _oracle(q, k, tau, invf, 0.5, 32)
+    k[:, 0, N - 1] *= 1e6
+    monkeypatch.setenv("STA_SCREEN_PASS1", screen)
+    votes, _, _ = _votes(q, k, tau, invf, 0.5, 32, False)
+    nt = (N - 1) // 32
+    assert (np.abs(votes - a["votes"])[:, :nt] <= a["band"][:, :nt]).all()
