@@ -613,11 +613,16 @@ hipError_t launch_abs_rope(int dtype, int D, const void* x, int64_t hs, int64_t 
 
 // Tiles (waves) per workgroup, unfused sweep.  A CU holds eight waves, two to a SIMD, by registers:
 // two workgroups of four tiles wait for each other's barriers less and leave less of a short call's
-// last round idle (16 heads x 12000, D 128, fp16: 3.01 ms against 3.23 with eight tiles; 32 x 16384
-// bf16: 10.0 either way).  fp32 stages twice the bytes a block, so long grids share each block among
-// eight tiles (32 heads x 4000, D 64: 670 us against 732; 8 heads x 4000, D 128: 811 against 731).
-constexpr int kStreamTiles = 4, kStreamTilesF32 = 8;
-constexpr int kStreamLongGrid = 2048;  // fp32: (head, tile) pairs, one wave each, that fill the chip
+// last round idle (fp16, D 128, block_n 32: 16 heads x 4000 603 us against 663 with eight tiles, 32 x
+// 4000 850 against 840, 32 x 12000 5.75 ms against 5.92).  Where a block stages twice the bytes, long
+// grids share each among eight tiles: fp32 (us with four and eight; D 128, 16 heads x 4000 869 and
+// 882, 20 heads 1093 and 923, 32 x 12000 11766 and 8107; D 64, 16 x 4000 495 and 509, 8 x 12000 1391
+// and 1434, 32 x 4000 672 and 607), and 16-bit rows of D 128 under block_n 64 (bf16, 8 x 4000 444 and
+// 445, 16 x 4000 603 and 583, 32 x 4000 799 and 727).
+constexpr int kStreamTiles = 4, kStreamTilesLong = 8;
+// (head, tile) pairs beyond which a grid is long; 0: four tiles always
+template <int DT, int D, int BN>
+constexpr int stream_long_grid() { return DT == DT_F32 ? 2048 : (D == 128 && BN == 64 ? 1024 : 0); }
 constexpr int kStreamTilesFused = 4;   // fused sweep: one wave per SIMD, the register room the
                                        // selection fragments need
 
@@ -639,7 +644,7 @@ constexpr size_t stream_lds_t(bool fused) {
   if constexpr (stream_fused<DT, D, BN>()) {
     if (fused) return StreamCfg<DT, D, BN, kStreamTilesFused, true>::lds_bytes;
   }
-  return StreamCfg<DT, D, BN, DT == DT_F32 ? kStreamTilesF32 : kStreamTiles, false>::lds_bytes;
+  return StreamCfg<DT, D, BN, (stream_long_grid<DT, D, BN>() > 0 ? kStreamTilesLong : kStreamTiles), false>::lds_bytes;
 }
 
 size_t stream_lds_bytes(int dtype, int D, int BN, bool fused) {
@@ -669,8 +674,9 @@ static hipError_t launch_stream_t(const StreamArgs& a, hipStream_t st) {
     if (a.qfrag) return launch_stream_g<DT, D, BN, kStreamTilesFused, true>(a, st);
   }
   if (!a.bits) return hipErrorInvalidValue;
-  if constexpr (DT == DT_F32) {
-    if ((int64_t)a.H * a.nt > kStreamLongGrid) return launch_stream_g<DT, D, BN, kStreamTilesF32, false>(a, st);
+  constexpr int LONG = stream_long_grid<DT, D, BN>();
+  if constexpr (LONG > 0) {
+    if ((int64_t)a.H * a.nt > LONG) return launch_stream_g<DT, D, BN, kStreamTilesLong, false>(a, st);
   }
   return launch_stream_g<DT, D, BN, kStreamTiles, false>(a, st);
 }

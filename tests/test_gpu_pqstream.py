@@ -357,9 +357,11 @@ def test_pqs_decode_rejects_bad_block_n():
 
 
 @pytest.mark.parametrize("dt,H,N,D,block_n", [(torch.float32, 2, 1283, 64, 64), (torch.float32, 24, 2780, 64, 32),
-                                              (torch.float16, 3, 257, 128, 64), (torch.bfloat16, 8, 33, 64, 32)])
+                                              (torch.float16, 3, 257, 128, 64), (torch.bfloat16, 8, 33, 64, 32),
+                                              (torch.bfloat16, 33, 1000, 128, 64)])
 def test_stream_workgroup_sizes_and_mask_edges(dt, H, N, D, block_n):
-    """Both workgroup sizes of the fp32 sweep (24 heads x 87 tiles and more take eight tiles), the
+    """Both workgroup sizes of the fp32 sweep (24 heads x 87 tiles and more take eight tiles) and of the
+    16-bit one at D 128 and block_n 64 (33 x 32 and more), the
     bit-transposed masks at 32- and 64-key blocks, and tiles and blocks cut by the last row."""
     import _sta_native as native
     from synthetic import base_inv_freq, planted_inputs
