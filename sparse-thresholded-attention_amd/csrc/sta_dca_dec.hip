@@ -319,7 +319,8 @@ __global__ __launch_bounds__(DCA_DEC_BK) void dca_dec_score16_kernel(DcaDecArgs 
 // HBM-bound: every value row is read once for GP heads, D / 8 lanes a row in 16-byte pieces.  The first PF rows of a lane are requested
 // before the block partials are reduced and the weights taken, so they arrive meanwhile.  65535
 // keys, 32 query / 8 kv heads, D 128, bf16: 29.5 us, 4.6 TB/s (one workgroup a query head with
-// 2-byte loads: 220 us; all 16 rows of a lane in flight, two workgroups a CU: 50 us).
+// 2-byte loads: 220 us); a call 60.8 us, with all 16 rows of a lane in flight 72.6 at two workgroups
+// a CU, and 197 at four, where they spill.
 // ------------------------------------------------------------------------------------------
 template <int DT, int D, int GP>
 __global__ __launch_bounds__(DCA_DEC_BK, DT != DT_F32 ? 4 : 1) void dca_dec_pv_kernel(DcaDecArgs a) {
