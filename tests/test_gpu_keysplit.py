@@ -136,30 +136,30 @@ def test_concentrated_scores_keep_three_products(dt, tile, monkeypatch):
     assert np.array_equal(ma, mb) and np.array_equal(va, vb), f"{int((va != vb).sum())} vote entries differ"
 
 
-@pytest.mark.parametrize("H,Hkv,N,D,dt", [(2, 1, 1500, 128, torch.float32), (3, 3, 700, 64, torch.bfloat16),
-                                          (4, 2, 8300, 64, torch.float32)])
-@pytest.mark.parametrize("score", ["freq", "margin", "expmass"])
+@pytest.mark.parametrize("H,Hkv,N,D,dt,scores", [
+    (2, 1, 1500, 128, torch.float32, ("freq", "margin", "expmass")), (4, 2, 8300, 64, torch.float32, ("freq", "margin", "expmass")),
+    (3, 3, 700, 64, torch.bfloat16, ("margin", "expmass")),           # the row-count instance has no fp6 pass 2
+])
 @pytest.mark.parametrize("pieces", ["0", "1", "3", "7"])
-def test_groups_that_the_screen_gave_up(H, Hkv, N, D, dt, score, pieces, monkeypatch):
+def test_groups_that_the_screen_gave_up(H, Hkv, N, D, dt, scores, pieces, monkeypatch):
     """The first half of one kv head's keys repeats one key: the screen gives up where rows see little
     else, and the split pass 2 takes the maxima that a sweep of those row groups left.  The row-count
     instance stays whole and sweeps inside.  (Whole plain votes sweep 512 rows where one half of them
     was given up, the row-count instance 256: there all keys of the head are the same.)"""
     import _sta_native as native
-    if dt != torch.float32 and score == "freq":
-        pytest.skip("whole instances have no fp6 pass 2")
-    say(f"screen gave up: H={H} Hkv={Hkv} N={N} D={D} {dt} {score} pieces={pieces}")
-    q, k, _, invf, tau = _inputs(H, Hkv, N, D, dt, 53)
-    k[:, 0, : N if score == "freq" and pieces in "01" else N // 2] = k[:, 0, :1]
     monkeypatch.setenv("STA_SCREEN_PASS1", "1")
     monkeypatch.setenv("STA_SCORE_PIECES", pieces)
-    got = []
-    for counts in (False, True):
-        r = native.select_vote(q, k, tau, invf, 0.0, 1.0, 1.0 / math.sqrt(D), 32, want_row_counts=counts, select_score=score)
-        torch.cuda.synchronize()
-        got.append([r[i].cpu().numpy() for i in range(len(r)) if i != 1])
-    for a, b in zip(*got):
-        assert np.array_equal(a, b), f"{int((a != b).sum())} of {a.size} entries differ"
+    for score in scores:
+        say(f"screen gave up: H={H} Hkv={Hkv} N={N} D={D} {dt} {score} pieces={pieces}")
+        q, k, _, invf, tau = _inputs(H, Hkv, N, D, dt, 53)
+        k[:, 0, : N if score == "freq" and pieces in "01" else N // 2] = k[:, 0, :1]
+        got = []
+        for counts in (False, True):
+            r = native.select_vote(q, k, tau, invf, 0.0, 1.0, 1.0 / math.sqrt(D), 32, want_row_counts=counts, select_score=score)
+            torch.cuda.synchronize()
+            got.append([r[i].cpu().numpy() for i in range(len(r)) if i != 1])
+        for a, b in zip(*got):
+            assert np.array_equal(a, b), f"{score}: {int((a != b).sum())} of {a.size} entries differ"
 
 
 def test_tied_scores_cost_one_sweep():
@@ -361,3 +361,37 @@ def test_one_key_far_out_of_few(N, screen, dt, monkeypatch):
     votes, _, _ = _votes(q, k, tau, invf, 0.5, 32, False)
     nt = (N - 1) // 32
     assert (np.abs(votes - a["votes"])[:, :nt] <= a["band"][:, :nt]).all()
+
+
+@pytest.mark.parametrize("screen", ["0", "1"])
+@pytest.mark.parametrize("score", ["freq", "expmass"])
+def test_swept_groups_in_a_graph(screen, score, monkeypatch):
+    """A graph over keys that tie and keys that do not, in turn, and a tau that calls for three products
+    in between: each replay starts from its own flags and maxima and gives the eager call's outputs."""
+    import _sta_native as native
+    H, N, D = 3, 1500, 64
+    say(f"graph: screen={screen} {score}")
+    monkeypatch.setenv("STA_SCREEN_PASS1", screen)
+    monkeypatch.setenv("STA_SCORE_PIECES", "3")
+    q, k, v, invf, _ = _inputs(H, H, N, D, torch.float32, 79)
+    tied = k.clone()
+    tied[:, 1] = tied[:, 1, :1]
+    kw = dict(pct=30.0, tile=64, k_max=256, want_votes=True, select_score=score)
+    kb, tb = k.clone(), torch.full((H,), 5.0, device=DEV)
+    plan = native.NoallocPlan(q, kb, v, tb, invf, 0.0, 1.0, invf, 0.5, 1.0, **kw)
+    plan.run()
+    torch.cuda.synchronize()
+    inputs = [(k, 5.0), (tied, 5.0), (k, 0.0), (tied, 0.0), (k, 5.0), (tied, 5.0)]
+    refs = [native.shared_attention(q, keys, v, torch.full((H,), t), invf, 0.0, 1.0, invf, 0.5, 1.0, **kw) for keys, t in inputs]
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        plan.run()
+    torch.cuda.synchronize()
+    for i, ((keys, t), ref) in enumerate(zip(inputs, refs)):
+        kb.copy_(keys)
+        tb.fill_(t)
+        g.replay()
+        torch.cuda.synchronize()
+        for name in ("votes", "idx", "kept_size", "out"):
+            assert torch.equal(plan.out[name], ref[name]), f"replay {i}: {name}"
